@@ -362,8 +362,9 @@ int pf_xfer_route_shape(pf_xfer* xfer, uint32_t route, uint32_t* threads,
  * workgroups take tiles from a queue in order (best over the host link,
  * whose bandwidth the XCDs do not share fairly: the queue keeps tiles, and
  * a marked load's layers, finishing in order, and few requests in flight
- * keep the link at its peak).  Marked launches always run queued (at
- * PF_LOAD_HOST_DEFAULT_GRID when their route says 0).  pf_xfer_set_max_grid
+ * keep the link at its peak).  Marked launches out of pinned host memory
+ * always run queued (at PF_LOAD_HOST_DEFAULT_GRID when their route says 0);
+ * marked copies between device buffers have a workgroup per 8 or 32 KiB.  pf_xfer_set_max_grid
  * caps both kinds.  Every route may run queued: the staged mode's two
  * streams each have a queue of their own, and a queued launch leaves its
  * queue empty. */

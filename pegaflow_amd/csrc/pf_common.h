@@ -55,9 +55,15 @@ struct SignalTargets {
   uint32_t count;
 };
 
-// The layers of one marking launch: chunks [chunk_start[g], chunk_start[g+1])
-// of the launch belong to call layer layer[g] (every group non-empty);
-// counters[layer] counts finished tiles and is 0 between launches.
+// A layer's counter of finished tiles or units, 0 between launches:
+// counters[layer * kCounterStride].  Each has a 128-byte line of its own:
+// the adds of one line run one after another, and those of the layers that
+// a launch has in flight run side by side.
+constexpr uint32_t kCounterStride = 32;
+
+// The layers of one marking queued launch: chunks [chunk_start[g],
+// chunk_start[g+1]) of the launch belong to call layer layer[g] (every group
+// non-empty).
 struct LayerMarks {
   const uint32_t* chunk_start;  // n + 1 entries, device memory
   const uint32_t* layer;        // n entries, device memory
@@ -66,19 +72,51 @@ struct LayerMarks {
   SignalTargets targets;
 };
 
-// The layers of one marked scatter of a staged slice (passed by value, so
-// the kernel reads them from its arguments): chunks [chunk_start[g],
-// chunk_start[g+1]) of the launch belong to call layer layer[g], for g < n
-// (every group non-empty, n <= kSliceMarkLayers).  tiles[g] is the layer's
-// tile count over all the launches that copy it (a layer may span slices:
-// counters[layer] adds up across them and the launch that reaches the count
-// marks the layer), or 0 for a layer marked otherwise (not counted).
+// A marked copy between device buffers works in units of up to 64 *
+// kMarkedUnroll 16-byte words of one chunk, one wave each; a workgroup of
+// kMarkedThreads takes up to 4 * loops consecutive units of one layer.
+constexpr uint32_t kMarkedThreads = 256;
+constexpr uint32_t kMarkedUnroll = 2;
+struct MarkedShape {
+  uint32_t units_per_chunk;
+  uint32_t wg_units;  // units of one workgroup
+};
+inline MarkedShape marked_shape(uint64_t chunk_bytes, uint64_t launch_chunks) {
+  const uint64_t unit = 64ull * kMarkedUnroll * 16;
+  // 32 KiB a workgroup, and 8 KiB in launches too small to fill the chip
+  // with those (see copy_chunks_marked_kernel).
+  const uint32_t loops = launch_chunks * chunk_bytes >= (32ull << 20) ? 4 : 1;
+  return {static_cast<uint32_t>((chunk_bytes + unit - 1) / unit), kMarkedThreads / 64 * loops};
+}
+// Workgroups of a layer's `chunks` chunks in one launch.
+inline uint64_t marked_workgroups(const MarkedShape& s, uint64_t chunks) {
+  return (chunks * s.units_per_chunk + s.wg_units - 1) / s.wg_units;
+}
+
+// The layers of one marked copy between device buffers, as a table in device
+// memory (any number of layers) ...
+struct MarkTable {
+  const uint32_t* wg_start;     // n + 1 entries: the launch's first workgroup of each layer
+  const uint32_t* chunk_start;  // n + 1 entries: the launch's first chunk of each layer
+  const uint32_t* layer;        // n entries
+  uint32_t n;
+  uint32_t* counters;
+  SignalTargets targets;
+};
+
+// ... or passed by value, so the kernel reads them from its arguments (a
+// slice of a staged load, n <= kSliceMarkLayers; every group non-empty).
+// units[g] is the layer's unit count over all the launches that copy it (a
+// layer may span slices: its counter adds up across them and the launch that
+// reaches the count marks the layer), or 0 for a layer marked otherwise (not
+// counted).  wg_start is filled in by launch_copy_chunks_marked.
 constexpr uint32_t kSliceMarkLayers = 8;
 struct SliceMarks {
   uint32_t n;
+  uint32_t wg_start[kSliceMarkLayers + 1];
   uint32_t chunk_start[kSliceMarkLayers + 1];
   uint32_t layer[kSliceMarkLayers];
-  uint32_t tiles[kSliceMarkLayers];
+  uint32_t units[kSliceMarkLayers];
   uint32_t* counters;
   SignalTargets targets;
 };
@@ -104,12 +142,16 @@ hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
                                     uint32_t grid, const LayerMarks* marks,
                                     uint32_t* queue, uint32_t* n_tiles, hipStream_t stream);
-// A marked copy between device buffers with a fixed workgroup -> tile map
-// (16-byte aligned chunks): each finished layer of `marks` is marked.
+// A marked copy between device buffers (16-byte aligned chunks): each finished
+// layer of the marks is marked.  At most max_grid workgroups (0: no cap).  The
+// table's n_wg workgroups and its entries are those of marked_shape(chunk_bytes,
+// n_chunks) over its layers.
 hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks,
-                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
-                                     uint32_t grid, const SliceMarks& marks,
+                                     uint64_t chunk_bytes, uint32_t max_grid, SliceMarks marks,
                                      hipStream_t stream);
+hipError_t launch_copy_chunks_mark_table(const ChunkDesc* d_descs, uint32_t n_chunks,
+                                         uint64_t chunk_bytes, uint32_t n_wg, uint32_t max_grid,
+                                         const MarkTable& marks, hipStream_t stream);
 hipError_t launch_mark_layers(const LayerList& list, const SignalTargets& t,
                               hipStream_t stream);
 hipError_t launch_wait_word(uint64_t word, uint64_t value, uint64_t max_ticks,

@@ -118,7 +118,7 @@ __device__ __forceinline__ void tile_done(const LayerMarks& m, uint32_t c,
   }
   const uint32_t layer = m.layer[lo];
   const uint32_t tiles = (m.chunk_start[lo + 1] - m.chunk_start[lo]) * tiles_per_chunk;
-  uint32_t* cnt = m.counters + layer;
+  uint32_t* cnt = m.counters + layer * kCounterStride;
   const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
   if (prev + 1 == tiles) {
@@ -128,111 +128,114 @@ __device__ __forceinline__ void tile_done(const LayerMarks& m, uint32_t c,
   }
 }
 
-// tile_done for k tiles of group g of a slice's marks at once, counted
-// toward the layer's tiles over all its launches.  The group table lives in
-// the kernel's arguments; it is read with constant indices only, so it
-// stays in scalar registers.
-__device__ __forceinline__ void slice_tiles_done(const SliceMarks& m, uint32_t g, uint32_t k) {
-  uint32_t layer = 0, tiles = 0;
-#pragma unroll
-  for (uint32_t i = 0; i < kSliceMarkLayers; ++i)
-    if (i == g) {
-      layer = m.layer[i];
-      tiles = m.tiles[i];
-    }
-  if (tiles == 0) return;  // marked by another kernel
-  uint32_t* cnt = m.counters + layer;
-  const uint32_t prev = __hip_atomic_fetch_add(cnt, k, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-  if (prev + k == tiles) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    write_marks(m.targets, layer);
+// The layer that workgroup `wg` of a marked copy belongs to: its first
+// workgroup and chunk, its chunks in this launch, its units over all launches
+// (0: not counted) and its index in the call.
+struct MarkGroup {
+  uint32_t wg_start, chunk_start, chunks, units, layer;
+};
+
+// wg < wg_start[n]; the search keeps wg_start[lo] <= wg < wg_start[hi].
+__device__ __forceinline__ MarkGroup mark_group(const MarkTable& m, uint32_t wg,
+                                                uint32_t units_per_chunk) {
+  uint32_t lo = 0, hi = m.n;
+  while (hi - lo > 1) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (m.wg_start[mid] <= wg) lo = mid;
+    else hi = mid;
   }
+  const uint32_t chunks = m.chunk_start[lo + 1] - m.chunk_start[lo];
+  return {m.wg_start[lo], m.chunk_start[lo], chunks, chunks * units_per_chunk, m.layer[lo]};
 }
 
-// The group of chunk c: the last g < n with chunk_start[g] <= c.
-__device__ __forceinline__ uint32_t slice_group_of(const SliceMarks& m, uint32_t c) {
-  uint32_t g = 0;
+// The table lives in the kernel's arguments: read with constant indices only,
+// so it stays in scalar registers.
+__device__ __forceinline__ MarkGroup mark_group(const SliceMarks& m, uint32_t wg, uint32_t) {
+  MarkGroup g{m.wg_start[0], m.chunk_start[0], m.chunk_start[1] - m.chunk_start[0], m.units[0],
+              m.layer[0]};
 #pragma unroll
   for (uint32_t i = 1; i < kSliceMarkLayers; ++i)
-    if (i < m.n && m.chunk_start[i] <= c) g = i;
+    if (i < m.n && m.wg_start[i] <= wg)
+      g = {m.wg_start[i], m.chunk_start[i], m.chunk_start[i + 1] - m.chunk_start[i], m.units[i],
+           m.layer[i]};
   return g;
 }
 
-// A marked copy between device buffers (the staged load's scatter of a
-// slice whose layers it reports itself): a fixed map like
-// copy_chunks_v16_kernel.  Workgroup w copies tiles w, w + grid, ..., which
-// run through the launch's layers in order, and reports the tiles it
-// finished of a layer once, when it moves on to the next layer or ends, not
-// once per tile: one counter takes one add at a time, and per-tile adds
-// (2,560 for a 40 MiB layer, in a queued launch) held such a copy at a
-// fraction of HBM rate.
+// 16 bytes at base + 16 * lane, written through the XCD's L2 to the device's
+// coherence point (the sc1 policy of an agent-scope store, which the language
+// offers for at most 8 bytes at a time).  `base` is the same for the whole
+// wave; `bytes` bounds the store: lanes past it write nothing.
+__device__ __forceinline__ void store16_through(uint64_t base, uint32_t bytes, uint32_t lane,
+                                                u32x4 v) {
+  constexpr int kSc1 = 16;
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<void*>(base), 0, static_cast<int>(bytes), 0x00027000);
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, static_cast<int>(lane * 16), 0, kSc1);
+}
+
+// A marked copy between device buffers: the device-sourced marked load (one
+// launch over its layers, table in device memory) and the staged load's
+// scatter of a slice whose layers it reports itself (table in the arguments).
 //
-// Visibility differs from the marking protocol above: the bytes are stored
-// as ordinary (write-back) stores, and before a workgroup reports a layer,
-// every wave's stores are acknowledged (s_waitcnt 0), the workgroup meets
-// at its barrier, and one lane issues an agent-scope release fence, which
-// writes its XCD's L2 back to the device's coherence point; then it adds to
-// the counter.  The finishing workgroup acquires and writes the marks as
-// above.  A fence writes back the whole L2, so it pays per workgroup, not
-// per store: with 128 workgroups a 40 MiB layer took 24.8 us, against 35.9
-// with write-through stores and 73 with 1,280 workgroups.  The report
-// condition depends only on the tile index, so it is uniform across the
-// workgroup and its barrier is reached by every lane.
-template <int UNROLL, bool NTL>
-__global__ void __launch_bounds__(1024)
-copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, uint32_t tiles_per_chunk,
-                          uint32_t n_tiles, uint32_t chunk16, SliceMarks marks) {
-  const uint32_t stride = blockDim.x;
-  const uint32_t tile_elems = stride * UNROLL;
-  uint32_t group = 0, done = 0;
-  for (uint32_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    const uint32_t c = t / tiles_per_chunk;
-    const uint32_t g = slice_group_of(marks, c);
-    if (done > 0 && g != group) {
-      __builtin_amdgcn_s_waitcnt(0);  // every store of this wave acknowledged
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        slice_tiles_done(marks, group, done);
-      }
-      done = 0;
-    }
-    group = g;
-    const uint32_t tile = t - c * tiles_per_chunk;
-    const ChunkDesc d = descs[c];
-    const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src);
-    g_u32x4* __restrict__ dst = reinterpret_cast<g_u32x4*>(d.dst);
-    const uint32_t tile_base = tile * tile_elems;
-    const uint32_t base = tile_base + threadIdx.x;
-    u32x4 v[UNROLL];
-    if (tile_base + tile_elems <= chunk16) {
-      // Every load of the tile in flight before its stores.
+// Bound by HBM and by the reports.  A unit is 64 lanes x UNROLL words of one
+// chunk and belongs to one wave, so a chunk of any size wastes at most part of
+// its last unit.  Workgroup w copies the consecutive units of one layer that
+// its index gives it and then adds their number to the layer's counter, once:
+// adds to one counter run one after another (about 40 ns), so one per 4 KiB
+// doubled the time of the whole copy, and one per 32 KiB costs 5-25% of it.
+// Workgroups start in index order, so the layers land in order.
+//
+// Visibility: as in the marking protocol above, with 16-byte write-through
+// stores.  They run at the rate of ordinary ones (288 MB of 36 KiB chunks 93
+// us, ordinary 97, non-temporal 105-115), so no L2 has to be written back
+// before a report.  The per-workgroup release fence that this replaces allowed
+// only 128 workgroups: a 40 MiB layer took 24 us, here 17; and 61 layers of
+// 4.7 MB, one launch and one marking kernel each before, took 450 us, here
+// 120 in one launch.
+template <int UNROLL, class Marks>
+__global__ void __launch_bounds__(kMarkedThreads)
+copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape,
+                          uint32_t chunk16, uint32_t n_wg, Marks marks) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr uint32_t kWaves = kMarkedThreads / 64;
+  for (uint32_t wg = blockIdx.x; wg < n_wg; wg += gridDim.x) {
+    const MarkGroup g = mark_group(marks, wg, shape.units_per_chunk);
+    const uint32_t group_units = g.chunks * shape.units_per_chunk;
+    const uint32_t first = (wg - g.wg_start) * shape.wg_units;
+    const uint32_t left = group_units - first;
+    const uint32_t mine = left < shape.wg_units ? left : shape.wg_units;
+    for (uint32_t i = wave; i < mine; i += kWaves) {
+      const uint32_t unit = first + i;
+      const uint32_t c = unit / shape.units_per_chunk;
+      const uint32_t e0 = (unit - c * shape.units_per_chunk) * (64u * UNROLL);
+      const ChunkDesc d = descs[g.chunk_start + c];
+      const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src) + e0;
+      const uint32_t words = chunk16 - e0;  // of this unit and what follows it
+      u32x4 v[UNROLL];
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) v[u] = load16<NTL>(src + base + u * stride);
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) store16<true>(dst + base + u * stride, v[u]);
-    } else {
+      for (int u = 0; u < UNROLL; ++u)
+        if (u * 64u + lane < words) v[u] = load16<true>(src + u * 64u + lane);
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
-        const uint32_t e = base + u * stride;
-        if (e < chunk16) v[u] = load16<NTL>(src + e);
-      }
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        const uint32_t e = base + u * stride;
-        if (e < chunk16) store16<true>(dst + e, v[u]);
+        if (u * 64u >= words) break;
+        const uint32_t n = words - u * 64u;
+        store16_through(d.dst + (static_cast<uint64_t>(e0) + u * 64u) * 16u,
+                        (n < 64u ? n : 64u) * 16u, lane, v[u]);
       }
     }
-    ++done;
-  }
-  if (done > 0) {
-    __builtin_amdgcn_s_waitcnt(0);
+    if (g.units == 0) continue;  // marked by another kernel (uniform: no barrier is missed)
+    __builtin_amdgcn_s_waitcnt(0);  // every store of this wave acknowledged
     __syncthreads();
     if (threadIdx.x == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      slice_tiles_done(marks, group, done);
+      uint32_t* cnt = marks.counters + g.layer * kCounterStride;
+      const uint32_t prev = __hip_atomic_fetch_add(cnt, mine, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+      if (prev + mine == g.units) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        write_marks(marks.targets, g.layer);
+      }
     }
   }
 }
@@ -553,49 +556,62 @@ hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
   return hipGetLastError();
 }
 
-template <int UNROLL>
-static void launch_marked(dim3 g, dim3 b, hipStream_t stream, bool ntl, const ChunkDesc* d,
-                          uint32_t tpc, uint32_t ntiles, uint32_t c16, const SliceMarks& m) {
-  if (ntl)
-    hipLaunchKernelGGL((copy_chunks_marked_kernel<UNROLL, true>), g, b, 0, stream, d, tpc,
-                       ntiles, c16, m);
-  else
-    hipLaunchKernelGGL((copy_chunks_marked_kernel<UNROLL, false>), g, b, 0, stream, d, tpc,
-                       ntiles, c16, m);
+// Every unit of a marked launch lies in its chunk: chunk16 < 2^31, and the
+// units of a launch are counted in 32 bits.
+static bool marked_fits(const MarkedShape& s, uint32_t n_chunks, uint64_t chunk_bytes,
+                        uint64_t n_wg) {
+  return chunk_bytes % 16 == 0 && chunk_bytes / 16 < (1ull << 31) &&
+         static_cast<uint64_t>(n_chunks) * s.units_per_chunk + s.wg_units <= 0xffffffffull &&
+         n_wg > 0 && n_wg + kMaxGrid <= 0xffffffffull;
+}
+
+template <class Marks>
+static hipError_t launch_marked(const ChunkDesc* d_descs, uint64_t chunk_bytes,
+                                const MarkedShape& s, uint32_t n_wg, uint32_t max_grid,
+                                const Marks& marks, hipStream_t stream) {
+  uint32_t cap = max_grid ? max_grid : kMaxGrid;
+  if (cap > kMaxGrid) cap = kMaxGrid;
+  hipLaunchKernelGGL((copy_chunks_marked_kernel<kMarkedUnroll, Marks>),
+                     dim3(n_wg < cap ? n_wg : cap), dim3(kMarkedThreads), 0, stream, d_descs, s,
+                     static_cast<uint32_t>(chunk_bytes / 16), n_wg, marks);
+  return hipGetLastError();
 }
 
 hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks,
-                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
-                                     uint32_t grid, const SliceMarks& marks,
+                                     uint64_t chunk_bytes, uint32_t max_grid, SliceMarks marks,
                                      hipStream_t stream) {
   if (n_chunks == 0 || chunk_bytes == 0) return hipSuccess;
-  if (threads == 0 || threads > 1024 || threads % 64 != 0 || grid == 0 || grid > kMaxGrid)
-    return hipErrorInvalidValue;
   if (marks.n == 0 || marks.n > kSliceMarkLayers || !marks.counters ||
       marks.targets.count == 0 || marks.targets.count > kMaxSignalTargets ||
       marks.chunk_start[0] != 0 || marks.chunk_start[marks.n] != n_chunks)
     return hipErrorInvalidValue;
-  const bool ntl = (unroll & PF_KERNEL_NT_LOADS) != 0;
-  unroll &= 0xffu;
-  uint32_t tpc = 0, ntiles = 0, c16 = 0;
-  if (!tile_geometry(n_chunks, chunk_bytes, threads, unroll, &tpc, &ntiles, &c16))
-    return hipErrorInvalidValue;
-  // Groups in chunk order, each counting at least its own tiles.
-  for (uint32_t g = 0; g < marks.n; ++g)
-    if (marks.chunk_start[g + 1] <= marks.chunk_start[g] ||
-        (marks.tiles[g] != 0 &&
-         static_cast<uint64_t>(marks.tiles[g]) <
-             static_cast<uint64_t>(marks.chunk_start[g + 1] - marks.chunk_start[g]) * tpc))
+  const MarkedShape s = marked_shape(chunk_bytes, n_chunks);
+  // Groups in chunk order, each counting at least its own units.
+  uint64_t wg = 0;
+  for (uint32_t g = 0; g < marks.n; ++g) {
+    if (marks.chunk_start[g + 1] <= marks.chunk_start[g]) return hipErrorInvalidValue;
+    const uint64_t chunks = marks.chunk_start[g + 1] - marks.chunk_start[g];
+    if (marks.units[g] != 0 && marks.units[g] < chunks * s.units_per_chunk)
       return hipErrorInvalidValue;
-  if (static_cast<uint64_t>(ntiles) + grid > 0xffffffffull) return hipErrorInvalidValue;
-  const dim3 g(grid < ntiles ? grid : ntiles), b(threads);
-  switch (unroll) {
-    case 1: launch_marked<1>(g, b, stream, ntl, d_descs, tpc, ntiles, c16, marks); break;
-    case 2: launch_marked<2>(g, b, stream, ntl, d_descs, tpc, ntiles, c16, marks); break;
-    case 4: launch_marked<4>(g, b, stream, ntl, d_descs, tpc, ntiles, c16, marks); break;
-    default: return hipErrorInvalidValue;
+    marks.wg_start[g] = static_cast<uint32_t>(wg);
+    wg += marked_workgroups(s, chunks);
   }
-  return hipGetLastError();
+  if (!marked_fits(s, n_chunks, chunk_bytes, wg)) return hipErrorInvalidValue;
+  marks.wg_start[marks.n] = static_cast<uint32_t>(wg);
+  return launch_marked(d_descs, chunk_bytes, s, static_cast<uint32_t>(wg), max_grid, marks,
+                       stream);
+}
+
+hipError_t launch_copy_chunks_mark_table(const ChunkDesc* d_descs, uint32_t n_chunks,
+                                         uint64_t chunk_bytes, uint32_t n_wg, uint32_t max_grid,
+                                         const MarkTable& marks, hipStream_t stream) {
+  if (n_chunks == 0 || chunk_bytes == 0) return hipSuccess;
+  if (marks.n == 0 || !marks.wg_start || !marks.chunk_start || !marks.layer || !marks.counters ||
+      marks.targets.count == 0 || marks.targets.count > kMaxSignalTargets)
+    return hipErrorInvalidValue;
+  const MarkedShape s = marked_shape(chunk_bytes, n_chunks);
+  if (!marked_fits(s, n_chunks, chunk_bytes, n_wg)) return hipErrorInvalidValue;
+  return launch_marked(d_descs, chunk_bytes, s, n_wg, max_grid, marks, stream);
 }
 
 hipError_t launch_mark_layers(const LayerList& list, const SignalTargets& t,

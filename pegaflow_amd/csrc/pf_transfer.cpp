@@ -291,23 +291,6 @@ constexpr uint64_t kScatterTrialMinBytes = 64ull << 20;  // time only launches t
 constexpr int kEngineSlots = 8;
 // Largest slice of a staged load that reports each layer's completion.
 constexpr uint64_t kLayeredLoadSlice = 64ull << 20;
-// Shape of a marked staged load's scatter that marks its slice's layers
-// itself (copy_chunks_marked_kernel): 512 threads, up to four non-temporal
-// 16-byte loads per lane (a 32 KiB chunk is one tile), 128 workgroups.
-// Each workgroup ends each of its layers with a release fence that writes
-// its XCD's L2 back, so fewer, busier workgroups win: measured on 40 MiB
-// layers of 32 KiB chunks, 24.8 us per layer with 128 workgroups and four
-// loads per lane, 25.1 with 256, 32 with 512, 73 with 1,280, 108 with one
-// workgroup per 8 KiB tile, 46 with 64.
-constexpr uint32_t kMarkedScatterThreads = 512;
-constexpr uint32_t kMarkedScatterGrid = 128;
-// Loads per lane for chunks of chunk_bytes: the tile covers a chunk of up to
-// 32 KiB, or 32 KiB of a larger one.
-static uint32_t marked_unroll(uint64_t chunk_bytes) {
-  const uint64_t c16 = chunk_bytes / 16;
-  return c16 >= 4u * kMarkedScatterThreads ? 4u : c16 >= 2u * kMarkedScatterThreads ? 2u : 1u;
-}
-
 struct ScatterTrial {
   hipEvent_t start = nullptr, stop = nullptr;
   uint64_t bytes = 0;       // bytes of the launch being timed
@@ -633,10 +616,9 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
 }
 
 // A marked copy between device buffers (16-byte aligned chunks) on the
-// context's stream with a fixed workgroup -> tile map: the staged load's
-// scatter of a slice whose layers it marks itself.
-int launch_marked_scatter(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes,
-                          const SliceMarks& m) {
+// context's stream: launch_it(descriptors, stream) issues it.
+template <class F>
+int launch_marked_copy(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, F launch_it) {
   if (n == 0) return PF_OK;
   if (int rc = check_launch_size(n, chunk_bytes)) return rc;
   std::pair<hipEvent_t, hipEvent_t>* tm = nullptr;
@@ -651,9 +633,7 @@ int launch_marked_scatter(pf_xfer* x, size_t first, size_t n, uint64_t chunk_byt
     PF_HIP(hipEventRecord(tm->first, x->stream));
   }
   (void)hipGetLastError();
-  const hipError_t e = launch_copy_chunks_marked(
-      x->desc_base + first, static_cast<uint32_t>(n), chunk_bytes, kMarkedScatterThreads,
-      marked_unroll(chunk_bytes) | PF_KERNEL_NT_LOADS, kMarkedScatterGrid, m, x->stream);
+  const hipError_t e = launch_it(x->desc_base + first, x->stream);
   if (e != hipSuccess) return hip_fail(e, "marked scatter kernel launch");
   if (tm) PF_HIP(hipEventRecord(tm->second, x->stream));
   x->last_kernels++;
@@ -673,14 +653,21 @@ int ensure_counters(pf_xfer* x, size_t num_layers) {
   x->d_queue[0] = x->d_queue[1] = nullptr;
   x->counters_cap = 0;
   // cap counters, then one 256-byte line per lane holding its tile queue.
-  const size_t words = cap + 128;
+  const size_t counts = cap * kCounterStride, words = counts + 128;
   PF_HIP(hipMalloc(reinterpret_cast<void**>(&x->d_counters), words * sizeof(uint32_t)));
   PF_HIP(hipMemsetAsync(x->d_counters, 0, words * sizeof(uint32_t), x->stream));
   PF_HIP(hipStreamSynchronize(x->stream));  // the link-side lane's first launch finds 0 too
-  x->d_queue[0] = x->d_counters + cap;
-  x->d_queue[1] = x->d_counters + cap + 64;
+  x->d_queue[0] = x->d_counters + counts;
+  x->d_queue[1] = x->d_counters + counts + 64;
   x->counters_cap = cap;
   return PF_OK;
+}
+
+// Descriptor slots that the mark tables of a call over num_layers layers take
+// at most, in up to two parts: a launch of n layers has up to 3n + 2 words, and
+// every layer may be a launch of its own.
+uint64_t mark_table_descs(uint32_t num_layers) {
+  return 5ull * num_layers * sizeof(uint32_t) / sizeof(ChunkDesc) + 2;
 }
 
 // Marks the given layers on the context's stream (after the work queued so far).
@@ -980,7 +967,7 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
     // is uploaded: growing the buffers later would wait for its copies.
     uint64_t bound = sp.n_desc;
     if (piped) {  // with the first layer's mark tables, when the kernel copies it
-      bound = 1 + 2 * ((2ull * num_layers + 1) * sizeof(uint32_t) / sizeof(ChunkDesc) + 1);
+      bound = 1 + mark_table_descs(num_layers);
       for (uint32_t li = 0; li < num_layers; ++li)
         bound += (pending && li >= head ? pending->max_blocks : layers[li].num_blocks) *
                  (layers[li].layout.segments ? layers[li].layout.segments : 1);
@@ -1124,9 +1111,8 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
         m.layer[m.n] = pc.layer;
         m.chunk_start[m.n + 1] = m.chunk_start[m.n] + static_cast<uint32_t>(pc.end - pc.begin);
         if (self_marked[pc.layer] == 1) {
-          const uint64_t tile = uint64_t(kMarkedScatterThreads) * marked_unroll(p.chunk_bytes);
-          const uint64_t tpc = (p.chunk_bytes / 16 + tile - 1) / tile;
-          m.tiles[m.n] = static_cast<uint32_t>(p.chunks.size() * tpc);
+          m.units[m.n] = static_cast<uint32_t>(
+              p.chunks.size() * marked_shape(p.chunk_bytes, st.n_chunks).units_per_chunk);
           counts = true;
         }
         ++m.n;
@@ -1134,7 +1120,11 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
       if (counts) {
         m.counters = x->d_counters;
         m.targets = *sig;
-        return launch_marked_scatter(x, st.desc_first, st.n_chunks, st.chunk_bytes, m);
+        return launch_marked_copy(
+            x, st.desc_first, st.n_chunks, st.chunk_bytes, [&](const ChunkDesc* d, hipStream_t s) {
+              return launch_copy_chunks_marked(d, static_cast<uint32_t>(st.n_chunks),
+                                               st.chunk_bytes, x->max_grid, m, s);
+            });
       }
     }
     return launch(x, st.desc_first, st.n_chunks, st.chunk_bytes, al16, is_save);
@@ -1377,7 +1367,7 @@ int staged(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers, bool is
     if (rc != PF_OK && slice_marks) {
       const hipError_t e1 = hipStreamSynchronize(x->stream);
       const hipError_t e2 =
-          e1 == hipSuccess ? hipMemset(x->d_counters, 0, num_layers * sizeof(uint32_t)) : e1;
+          e1 == hipSuccess ? hipMemset(x->d_counters, 0, num_layers * kCounterStride * sizeof(uint32_t)) : e1;
       if (e2 != hipSuccess) (void)hipGetLastError();
     }
     PF_HIP(hipEventRecord(x->staging_free, x->stream));
@@ -1541,6 +1531,7 @@ struct Step {
   bool aligned;
   size_t tab = 0;      // marked launch: u32 offset of its table in the aux area
   uint32_t groups = 0; // marked launch: non-empty layers in it
+  uint32_t wgs = 0;    // marked copy between device buffers: its workgroups (0: queued)
 };
 
 // desc_off > 0: a later part of one pipelined call.  Its descriptors go
@@ -1565,7 +1556,8 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
   // Without per-layer events, consecutive layers with the same chunk size and
   // alignment share one launch (marks keep per-layer completion inside it).
   std::vector<Step> steps;
-  std::vector<uint32_t> aux;  // marked launches: chunk_start[n+1], then layer[n]
+  // Marked launches: chunk_start[n+1], then layer[n], then (device copies) wg_start[n+1].
+  std::vector<uint32_t> aux;
   for (size_t li = 0; li < plans.size();) {
     const LayerPlan& p = plans[li];
     if (p.ordered) {
@@ -1574,33 +1566,44 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
       continue;
     }
     const bool al = chunks_aligned(p);
-    // Marks inside the launch cost nothing while the host link is the bound
-    // (sources in pinned memory) but slow an HBM-bound launch; loads from
-    // device memory are split per layer and marked after each launch.
+    // A marked launch is queued when its sources are pinned host memory, and
+    // a marked device copy when they are device memory: one launch holds
+    // layers of one kind.
     const bool host_src = !p.chunks.empty() && host_sourced(p, is_save);
-    const bool per_layer = layer_events || (sig && !p.chunks.empty() && !host_src);
     size_t lj = li + 1;
-    if (!per_layer) {
+    if (!layer_events) {
       while (lj < plans.size() && !plans[lj].ordered &&
              plans[lj].chunk_bytes == p.chunk_bytes &&
-             (plans[lj].chunks.empty() || (chunks_aligned(plans[lj]) == al &&
-                                           (!sig || host_sourced(plans[lj], is_save)))))
+             (plans[lj].chunks.empty() ||
+              (chunks_aligned(plans[lj]) == al &&
+               (!sig || host_sourced(plans[lj], is_save) == host_src))))
         ++lj;
     }
     Step st{li, lj, false, al};
-    if (sig && al && !per_layer) {
+    if (sig && al && !layer_events) {
       st.tab = aux.size();
-      uint32_t start = 0;
-      std::vector<uint32_t> ids;
+      size_t chunks = 0;
+      for (size_t k = li; k < lj; ++k) chunks += plans[k].chunks.size();
+      const MarkedShape shape = marked_shape(p.chunk_bytes, chunks);
+      std::vector<uint32_t> ids, wg_start;
+      uint64_t start = 0, wgs = 0;
       for (size_t k = li; k < lj; ++k) {
         if (plans[k].chunks.empty()) continue;
-        aux.push_back(start);
+        aux.push_back(static_cast<uint32_t>(start));
+        wg_start.push_back(static_cast<uint32_t>(wgs));
         ids.push_back(static_cast<uint32_t>(layer_base + k));
-        start += static_cast<uint32_t>(plans[k].chunks.size());
+        start += plans[k].chunks.size();
+        wgs += marked_workgroups(shape, plans[k].chunks.size());
       }
-      aux.push_back(start);
+      aux.push_back(static_cast<uint32_t>(start));
       aux.insert(aux.end(), ids.begin(), ids.end());
       st.groups = static_cast<uint32_t>(ids.size());
+      if (!host_src && wgs > 0) {
+        if (wgs > 0xffffffffull) return fail(PF_ERR_INVALID_ARGUMENT, "too many chunks");
+        aux.insert(aux.end(), wg_start.begin(), wg_start.end());
+        aux.push_back(static_cast<uint32_t>(wgs));
+        st.wgs = static_cast<uint32_t>(wgs);
+      }
     }
     steps.push_back(st);
     li = lj;
@@ -1646,25 +1649,42 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     }
     size_t n = 0;
     for (size_t k = st.li; k < st.lj; ++k) n += plans[k].chunks.size();
-    LayerMarks marks{};
     const bool marked = st.groups > 0;
-    if (marked) {
-      marks.chunk_start = d_aux + st.tab;
-      marks.layer = d_aux + st.tab + st.groups + 1;
-      marks.n = st.groups;
-      marks.counters = x->d_counters;
-      marks.targets = *sig;
-    }
-    // The launch shape follows the first non-empty layer's host side.
-    bool host_side = false;
-    for (size_t k = st.li; k < st.lj; ++k)
-      if (!plans[k].chunks.empty()) {
-        host_side = host_side_pinned(plans[k]);
-        break;
+    if (st.wgs > 0) {
+      MarkTable t{};
+      t.chunk_start = d_aux + st.tab;
+      t.layer = t.chunk_start + st.groups + 1;
+      t.wg_start = t.layer + st.groups;
+      t.n = st.groups;
+      t.counters = x->d_counters;
+      t.targets = *sig;
+      const uint64_t cb = plans[st.li].chunk_bytes;
+      if (int rc = launch_marked_copy(
+              x, first[st.li], n, cb, [&](const ChunkDesc* dd, hipStream_t s) {
+                return launch_copy_chunks_mark_table(dd, static_cast<uint32_t>(n), cb, st.wgs,
+                                                     x->max_grid, t, s);
+              }))
+        return rc;
+    } else {
+      LayerMarks marks{};
+      if (marked) {
+        marks.chunk_start = d_aux + st.tab;
+        marks.layer = d_aux + st.tab + st.groups + 1;
+        marks.n = st.groups;
+        marks.counters = x->d_counters;
+        marks.targets = *sig;
       }
-    if (int rc = launch(x, first[st.li], n, plans[st.li].chunk_bytes, st.aligned, is_save,
-                        host_side, marked ? &marks : nullptr))
-      return rc;
+      // The launch shape follows the first non-empty layer's host side.
+      bool host_side = false;
+      for (size_t k = st.li; k < st.lj; ++k)
+        if (!plans[k].chunks.empty()) {
+          host_side = host_side_pinned(plans[k]);
+          break;
+        }
+      if (int rc = launch(x, first[st.li], n, plans[st.li].chunk_bytes, st.aligned, is_save,
+                          host_side, marked ? &marks : nullptr))
+        return rc;
+    }
     if (layer_events && layer_events[st.li])
       PF_HIP(hipEventRecord(static_cast<hipEvent_t>(layer_events[st.li]), x->stream));
     if (sig) {
@@ -1721,10 +1741,10 @@ int kernel_pipelined(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layer
   if (int rc = plan_all(layers, head, is_save, &first)) return rc;
   for (uint32_t li = 0; li < head; ++li)
     apply_write_policy(layers[li], is_save, false, &first[li]);
-  // Room for every descriptor of the call and both parts' mark tables
-  // (at most 2L+1 words each), reserved before the first part is uploaded:
+  // Room for every descriptor of the call and both parts' mark tables,
+  // reserved before the first part is uploaded:
   // growing the buffers later would wait for the first copy.
-  uint64_t bound = 1 + 2 * ((2ull * num_layers + 1) * sizeof(uint32_t) / sizeof(ChunkDesc) + 1);
+  uint64_t bound = 1 + mark_table_descs(num_layers);
   for (uint32_t i = 0; i < num_layers; ++i)
     bound += (pending && i >= head ? pending->max_blocks : layers[i].num_blocks) *
              (layers[i].layout.segments ? layers[i].layout.segments : 1);

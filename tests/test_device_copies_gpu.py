@@ -1,0 +1,96 @@
+"""GPU tests of copies between device buffers at the edges of the kernels' tiles.
+
+A kernel-mode save into, or load out of, a buffer in device memory moves each
+chunk as units of one wave.  The sizes here sit at the edges of a unit (one
+wave's words, one more, one less), of a workgroup's share and of a launch.  The
+expected bytes are a numpy indexing of the same layout.
+"""
+
+import numpy as np
+import pytest
+
+from pegaflow_amd import _lib
+from pegaflow_amd.runtime import DeviceBuffer, PinnedBuffer
+from pegaflow_amd.transfer import (KVCacheRegistration, LayerTransfer, TransferContext,
+                                   block_array)
+
+pytestmark = pytest.mark.gpu
+
+
+class Layer:
+    """A KV tensor of ``nb`` blocks in ``segs`` segments of ``bpb`` bytes, and the
+    ``ids`` that move between it and a buffer holding a K and a V region."""
+
+    def __init__(self, nb, bpb, segs, ids, seed):
+        self.shape, self.ids = (segs, nb, bpb), np.asarray(ids, np.int64)
+        self.dev = DeviceBuffer((segs * nb * bpb + 7) // 8 * 8)
+        self.dev.fill_random(seed)
+        self.host = self.dev.download()
+        self.reg = KVCacheRegistration.create(self.dev.ptr, segs * nb * bpb, nb, bpb,
+                                              nb * bpb if segs == 2 else 0, segs)
+        self.nbytes = segs * len(self.ids) * bpb
+
+    def view(self, flat):
+        segs, nb, bpb = self.shape
+        return flat[:segs * nb * bpb].reshape(self.shape)
+
+    def transfer(self, base):
+        segs, _, bpb = self.shape
+        at = base + np.arange(len(self.ids), dtype=np.uint64) * np.uint64(bpb)
+        v = at + np.uint64(len(self.ids) * bpb) if segs == 2 else None
+        return LayerTransfer(self.reg, block_array(self.ids, at, v))
+
+    def packed(self):
+        return self.view(self.host)[:, self.ids].reshape(-1)
+
+    def restore(self, packed):
+        segs, _, bpb = self.shape
+        self.view(self.host)[:, self.ids] = packed.reshape(segs, len(self.ids), bpb)
+
+
+def make_layers(rng, bpb, segs, counts, nb):
+    return [Layer(nb, bpb, segs, rng.choice(nb, n, replace=False), 10 + i)
+            for i, n in enumerate(counts)]
+
+
+def bases(layers, base):
+    out = []
+    for l in layers:
+        out.append(base)
+        base += l.nbytes
+    return out
+
+
+# Segment sizes around a wave's words (1 KiB) and its unit (2 KiB), and one of
+# many units; layers of none, one and several blocks.
+MARKED = [(bpb, 2, (3, 0, 1, 17), 40, cap)
+          for bpb in (16, 1008, 1024, 1040, 2032, 2048, 2064, 8208, 36864) for cap in (0, 3)]
+# A launch large enough for the larger share of a workgroup, blocks-first and split.
+MARKED += [(32768, 2, (300, 301), 400, 0), (36864, 1, (511, 1, 512), 600, 0)]
+
+
+@pytest.mark.parametrize("bpb,segs,counts,nb,cap", MARKED)
+def test_marked_load_from_device_memory(gpu, bpb, segs, counts, nb, cap):
+    """One marked launch over the layers: every byte and every word, twice (the
+    layers' counters are 0 again after a launch)."""
+    rng = np.random.default_rng(bpb + cap)
+    layers = make_layers(rng, bpb, segs, counts, nb)
+    pool = DeviceBuffer(sum(l.nbytes for l in layers))
+    words, dev_words = PinnedBuffer(8 * len(layers)), DeviceBuffer(8 * len(layers))
+    words.array[:] = 0
+    dev_words.memset(0)
+    ctx = TransferContext(0)
+    ctx.set_max_grid(cap)
+    for value in (1, 2):
+        pool.fill_random(100 + value, nbytes=pool.nbytes // 8 * 8)
+        packed = pool.download()
+        ctx.load_layers_marked([l.transfer(b) for l, b in zip(layers, bases(layers, pool.ptr))],
+                               [(words.ptr, value, True), (dev_words.ptr, value, False)],
+                               _lib.MODE_KERNEL)
+        ctx.synchronize()
+        assert words.array.view(np.uint64).tolist() == [value] * len(layers)
+        assert dev_words.download().view(np.uint64).tolist() == [value] * len(layers)
+        for l, at in zip(layers, bases(layers, 0)):
+            l.restore(packed[at:at + l.nbytes])
+            assert np.array_equal(l.dev.download(), l.host)
+    ctx.close()
