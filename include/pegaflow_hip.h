@@ -309,9 +309,11 @@ pf_stream pf_xfer_stream(pf_xfer* xfer);
 int pf_xfer_synchronize(pf_xfer* xfer);
 /* Select the kernel's launch shape: threads per workgroup (64..1024, multiple
  * of 64) and 16-byte loads in flight per lane (1, 2, 4, 8 or 16), optionally
- * OR-ed with PF_KERNEL_NT_LOADS and/or PF_KERNEL_NT_STORES for non-temporal
- * (streaming) loads and stores.  0 keeps the current value.  Sets the shape
- * of every route; defaults below. */
+ * OR-ed with PF_KERNEL_NT_LOADS and/or PF_KERNEL_NT_STORES for streaming
+ * loads and stores (non-temporal; a fixed-map launch's stores are written
+ * through the L2 instead).  A fixed-map launch hands out work by the wave and
+ * runs in workgroups of at most 256 threads.  0 keeps the current value.  Sets
+ * the shape of every route; defaults below. */
 #define PF_KERNEL_NT_LOADS 0x100u
 #define PF_KERNEL_NT_STORES 0x200u
 #define PF_KERNEL_NONTEMPORAL (PF_KERNEL_NT_LOADS | PF_KERNEL_NT_STORES)
@@ -335,7 +337,7 @@ enum {
   PF_ROUTE_LOAD_HOST = 3    /* pinned host memory -> paged tensor           */
 };
 /* Per-route defaults (the fastest shapes measured on MI355X): HBM gathers
- * move 8 KiB tiles in round-robin order; scatters choose on evidence
+ * move 1 KiB a wave in round-robin order; scatters choose on evidence
  * (PF_KERNEL_AUTO); zero-copy saves 16 KiB tiles with streaming loads and
  * ordinary stores into host memory (2% faster than streaming both). */
 #define PF_SAVE_DEFAULT_THREADS 512u

@@ -10,11 +10,12 @@
 //   * save:    paged layer tensor -> pinned host (or HBM staging), a gather;
 //   * restore: pinned host (or HBM staging) -> paged layer tensor, a scatter.
 //
-// Work decomposition: a chunk is split into tiles of blockDim.x * UNROLL
-// 16-byte elements.  One workgroup copies one tile: every lane issues UNROLL
-// independent 16-byte loads (global_load_dwordx4) before its UNROLL stores,
-// so each wave keeps UNROLL * 1 KiB in flight — enough to cover HBM latency
-// and, for zero-copy, the much longer host-link read latency.  Consecutive
+// Work decomposition: copies between device buffers split a chunk into units
+// of 64 * UNROLL 16-byte elements, one wave each; copies over the host link
+// into tiles of blockDim.x * UNROLL elements, one workgroup each.  Every lane
+// issues UNROLL independent 16-byte loads (global_load_dwordx4) before its
+// UNROLL stores, so each wave keeps UNROLL * 1 KiB in flight — enough to cover
+// HBM latency and, for zero-copy, the much longer host-link read latency.  Consecutive
 // lanes touch consecutive 16-byte words, so every wave instruction covers one
 // contiguous 1 KiB span (fully coalesced).  No LDS: source and destination
 // share the same byte order within a chunk.
@@ -240,41 +241,63 @@ copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape
   }
 }
 
-template <int UNROLL, bool NTL, bool NTS>
-__global__ void __launch_bounds__(1024)
-copy_chunks_v16_kernel(const ChunkDesc* __restrict__ descs,
-                       uint32_t tiles_per_chunk, uint32_t n_tiles,
-                       uint32_t chunk16, uint32_t xcd_major) {
-  const uint32_t stride = blockDim.x;
-  const uint32_t tile_elems = stride * UNROLL;
-  const bool remap = xcd_major && gridDim.x == n_tiles;
-  for (uint32_t b = blockIdx.x; b < n_tiles; b += gridDim.x) {
-    const uint32_t t = tile_of(b, n_tiles, remap);
-    const uint32_t c = t / tiles_per_chunk;
-    const uint32_t tile = t - c * tiles_per_chunk;
+// The fixed-map copy: between device buffers, and the descriptor uploads.
+//
+// Bound by HBM.  A unit is 64 lanes x UNROLL words of one chunk and belongs to
+// one wave: wave w of the launch copies unit w, so chunks of any size keep
+// every lane busy but for part of a chunk's last unit.  (A workgroup per tile
+// of 512 threads left lanes idle on every chunk that 8 KiB do not divide:
+// 1.34 GB of 10 KiB chunks gathered at 5.1 TB/s, with units 6.1; 168 MB of 2
+// KiB chunks 5.1 and 5.8.)  Workgroups have at most 4 waves: with 8 the 32 KiB
+// chunks of the Llama prefix gather at 5.95 TB/s and scatter at 5.44, with 4
+// at 6.10 and 5.61.  Streaming stores (THROUGH) are written through the L2 and
+// may stay in the memory-side cache: non-temporal ones, which bypass it, were
+// as fast on 1.34 GB and 11-25% slower on 67-288 MB.
+constexpr uint32_t kFixedThreads = 256;
+
+template <int UNROLL, bool NTL, bool THROUGH>
+__global__ void __launch_bounds__(kFixedThreads)
+copy_chunks_v16_kernel(const ChunkDesc* __restrict__ descs, uint32_t units_per_chunk,
+                       uint32_t n_units, uint32_t chunk16, uint32_t xcd_major) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t waves = blockDim.x >> 6;
+  const uint32_t n_wg = (n_units + waves - 1) / waves;
+  const bool remap = xcd_major && gridDim.x == n_wg;
+  for (uint32_t b = blockIdx.x; b < n_wg; b += gridDim.x) {
+    const uint32_t unit = __builtin_amdgcn_readfirstlane(tile_of(b, n_wg, remap) * waves +
+                                                         (threadIdx.x >> 6));
+    if (unit >= n_units) continue;
+    const uint32_t c = unit / units_per_chunk;
+    const uint32_t e0 = (unit - c * units_per_chunk) * (64u * UNROLL);
     const ChunkDesc d = descs[c];
-    const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src);
-    g_u32x4* __restrict__ dst = reinterpret_cast<g_u32x4*>(d.dst);
-    const uint32_t tile_base = tile * tile_elems;
-    const uint32_t base = tile_base + threadIdx.x;
+    const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src) + e0;
+    g_u32x4* __restrict__ dst = reinterpret_cast<g_u32x4*>(d.dst) + e0;
+    const uint32_t words = chunk16 - e0;  // of this unit and what follows it
     u32x4 v[UNROLL];
-    if (tile_base + tile_elems <= chunk16) {
+    if (words >= 64u * UNROLL) {
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) v[u] = load16<NTL>(src + base + u * stride);
+      for (int u = 0; u < UNROLL; ++u) v[u] = load16<NTL>(src + u * 64u + lane);
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) store16<NTS>(dst + base + u * stride, v[u]);
+      for (int u = 0; u < UNROLL; ++u) {
+        if constexpr (THROUGH)
+          store16_through(d.dst + (static_cast<uint64_t>(e0) + u * 64u) * 16u, 1024u, lane, v[u]);
+        else
+          dst[u * 64u + lane] = v[u];
+      }
     } else {
-      // Partial last tile of a chunk: guarded per element.
+      // Partial last unit of a chunk: guarded per word.
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        const uint32_t e = base + u * stride;
-        if (e < chunk16) v[u] = load16<NTL>(src + e);
-      }
+      for (int u = 0; u < UNROLL; ++u)
+        if (u * 64u + lane < words) v[u] = load16<NTL>(src + u * 64u + lane);
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        const uint32_t e = base + u * stride;
-        if (e < chunk16) store16<NTS>(dst + e, v[u]);
-      }
+      for (int u = 0; u < UNROLL; ++u)
+        if (u * 64u + lane < words) {
+          if constexpr (THROUGH)
+            store16_through(d.dst + (static_cast<uint64_t>(e0) + u * 64u) * 16u, 1024u, lane,
+                            v[u]);
+          else
+            dst[u * 64u + lane] = v[u];
+        }
     }
   }
 }
@@ -404,35 +427,37 @@ copy_chunks_b1_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
 // Upper bound on workgroups per launch; larger tile counts loop.
 static constexpr uint32_t kMaxGrid = 1u << 20;
 
-template <int UNROLL, bool NTL, bool NTS>
+template <int UNROLL, bool NTL, bool THROUGH>
 static void launch_v16_nt(dim3 grid, dim3 block, hipStream_t stream, const ChunkDesc* d,
-                          uint32_t tpc, uint32_t n_tiles, uint32_t c16, uint32_t xcd) {
-  hipLaunchKernelGGL((copy_chunks_v16_kernel<UNROLL, NTL, NTS>), grid, block, 0, stream, d,
-                     tpc, n_tiles, c16, xcd);
+                          uint32_t upc, uint32_t n_units, uint32_t c16, uint32_t xcd) {
+  hipLaunchKernelGGL((copy_chunks_v16_kernel<UNROLL, NTL, THROUGH>), grid, block, 0, stream, d,
+                     upc, n_units, c16, xcd);
 }
 
 template <int UNROLL>
-static hipError_t launch_v16(const ChunkDesc* d_descs, uint32_t tiles_per_chunk,
-                             uint32_t n_tiles, uint32_t chunk16, uint32_t threads,
+static hipError_t launch_v16(const ChunkDesc* d_descs, uint32_t units_per_chunk,
+                             uint32_t n_units, uint32_t chunk16, uint32_t threads,
                              uint32_t flags, uint32_t max_grid, hipStream_t stream) {
   const uint32_t cap = max_grid ? max_grid : kMaxGrid;
-  const dim3 grid(n_tiles < cap ? n_tiles : cap), block(threads);
+  const uint32_t waves = threads / 64;
+  const uint32_t n_wg = (n_units + waves - 1) / waves;
+  const dim3 grid(n_wg < cap ? n_wg : cap), block(threads);
   const uint32_t xcd = (flags & PF_KERNEL_XCD_MAJOR) ? 1u : 0u;
   switch (flags & PF_KERNEL_NONTEMPORAL) {
     case 0:
-      launch_v16_nt<UNROLL, false, false>(grid, block, stream, d_descs, tiles_per_chunk, n_tiles,
+      launch_v16_nt<UNROLL, false, false>(grid, block, stream, d_descs, units_per_chunk, n_units,
                                           chunk16, xcd);
       break;
     case PF_KERNEL_NT_LOADS:
-      launch_v16_nt<UNROLL, true, false>(grid, block, stream, d_descs, tiles_per_chunk, n_tiles,
+      launch_v16_nt<UNROLL, true, false>(grid, block, stream, d_descs, units_per_chunk, n_units,
                                          chunk16, xcd);
       break;
     case PF_KERNEL_NT_STORES:
-      launch_v16_nt<UNROLL, false, true>(grid, block, stream, d_descs, tiles_per_chunk, n_tiles,
+      launch_v16_nt<UNROLL, false, true>(grid, block, stream, d_descs, units_per_chunk, n_units,
                                          chunk16, xcd);
       break;
     default:
-      launch_v16_nt<UNROLL, true, true>(grid, block, stream, d_descs, tiles_per_chunk, n_tiles,
+      launch_v16_nt<UNROLL, true, true>(grid, block, stream, d_descs, units_per_chunk, n_units,
                                         chunk16, xcd);
       break;
   }
@@ -512,15 +537,18 @@ hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
                        stream, d_descs, n_chunks, chunk_bytes);
     return hipGetLastError();
   }
-  uint32_t tpc = 0, ntl = 0, c16 = 0;
-  if (!tile_geometry(n_chunks, chunk_bytes, threads, unroll, &tpc, &ntl, &c16))
+  // The waves' units are the launch's tiles; workgroups of at most kFixedThreads.
+  if (threads > kFixedThreads) threads = kFixedThreads;
+  uint32_t upc = 0, units = 0, c16 = 0;
+  if (!tile_geometry(n_chunks, chunk_bytes, 64, unroll, &upc, &units, &c16) ||
+      units > 0xffffffffu - 16u)
     return hipErrorInvalidValue;
   switch (unroll) {
-    case 1: return launch_v16<1>(d_descs, tpc, ntl, c16, threads, flags, max_grid, stream);
-    case 2: return launch_v16<2>(d_descs, tpc, ntl, c16, threads, flags, max_grid, stream);
-    case 4: return launch_v16<4>(d_descs, tpc, ntl, c16, threads, flags, max_grid, stream);
-    case 8: return launch_v16<8>(d_descs, tpc, ntl, c16, threads, flags, max_grid, stream);
-    case 16: return launch_v16<16>(d_descs, tpc, ntl, c16, threads, flags, max_grid, stream);
+    case 1: return launch_v16<1>(d_descs, upc, units, c16, threads, flags, max_grid, stream);
+    case 2: return launch_v16<2>(d_descs, upc, units, c16, threads, flags, max_grid, stream);
+    case 4: return launch_v16<4>(d_descs, upc, units, c16, threads, flags, max_grid, stream);
+    case 8: return launch_v16<8>(d_descs, upc, units, c16, threads, flags, max_grid, stream);
+    case 16: return launch_v16<16>(d_descs, upc, units, c16, threads, flags, max_grid, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -345,10 +345,8 @@ struct pf_xfer {
   // End of a pipelined staged load's first layer, copied by the kernel.
   hipEvent_t head_done = nullptr;
   // Launch shapes per route (PF_ROUTE_*), the fastest measured on MI355X:
-  //   gather into HBM:   512 threads, one non-temporal 16 B load per lane
-  //                      (8 KiB tiles), round-robin tile order;
-  //   scatter:           512 threads, two non-temporal loads per lane (16 KiB
-  //                      tiles), XCD-major tile order;
+  //   gather into HBM:   one streaming 16 B load per lane, round-robin order;
+  //   scatter:           chosen between kScatterShapes;
   //   save to the host:  512 threads, two streaming loads per lane, ordinary
   //                      stores into host memory.
   uint32_t threads[4] = {PF_SAVE_DEFAULT_THREADS, PF_LOAD_DEFAULT_THREADS,

@@ -94,3 +94,32 @@ def test_marked_load_from_device_memory(gpu, bpb, segs, counts, nb, cap):
             l.restore(packed[at:at + l.nbytes])
             assert np.array_equal(l.dev.download(), l.host)
     ctx.close()
+
+
+# Chunks around a wave's words and its units at each number of loads per lane,
+# a last unit of one word, and launches of one chunk.
+FIXED = [(bpb, segs, n) for bpb in (16, 1008, 1024, 1040, 4096, 10240, 16400) for segs, n in
+         ((1, 1), (2, 37))]
+
+
+@pytest.mark.parametrize("bpb,segs,n", FIXED)
+def test_fixed_map_copies(gpu, bpb, segs, n):
+    """Gather and scatter at every shape of the fixed map, capped grids included."""
+    rng = np.random.default_rng(bpb + n)
+    (layer,) = make_layers(rng, bpb, segs, (n,), 64)
+    pool = DeviceBuffer(layer.nbytes)
+    ctx = TransferContext(0)
+    shapes = [(t, u | f) for t in (64, 512) for u in (1, 2, 4, 8, 16)
+              for f in (0, _lib.KERNEL_NONTEMPORAL, _lib.KERNEL_NT_STORES | _lib.KERNEL_XCD_MAJOR)]
+    for i, (threads, unroll) in enumerate(shapes):
+        ctx.set_kernel_shape(threads, unroll)
+        ctx.set_max_grid((0, 3)[i % 2])
+        pool.memset(0)
+        ctx.save_layers([layer.transfer(pool.ptr)], _lib.MODE_KERNEL)
+        assert np.array_equal(pool.download(), layer.packed()), f"gather {threads} {unroll:#x}"
+        pool.fill_random(i, nbytes=pool.nbytes // 8 * 8)
+        layer.restore(pool.download())
+        ctx.load_layers([layer.transfer(pool.ptr)], _lib.MODE_KERNEL)
+        ctx.synchronize()
+        assert np.array_equal(layer.dev.download(), layer.host), f"scatter {threads} {unroll:#x}"
+    ctx.close()
