@@ -76,11 +76,11 @@ __device__ __forceinline__ uint32_t tile_of(uint32_t b, uint32_t n, bool xcd_maj
 // visible to readers on other XCDs only once it has left that L2.  A
 // release fence at agent scope per workgroup would write the whole L2 back
 // every time (measured: 2.2x slower from pinned memory, 40x from HBM).
-// Instead the marking kernel stores its bytes as agent-scope relaxed atomic
-// stores, which write through the L2 to the device's coherence point (the
-// sc1 policy), and waits for every store's acknowledgement (s_waitcnt 0)
-// before the workgroup barrier; only then does one lane bump the counter
-// (an agent-scope atomic).  The finishing workgroup acquires at agent scope,
+// Instead the marking kernels store their bytes through the L2 to the device's
+// coherence point (store16_through: the sc1 policy that agent-scope stores
+// have) and wait for every store's acknowledgement (s_waitcnt 0) before the
+// workgroup barrier; only then does one lane bump the counter (an agent-scope
+// atomic).  The finishing workgroup acquires at agent scope,
 // puts the counter back to 0 (ready for the next launch on the stream) and
 // writes the marks as release stores, at system scope for host memory.  A
 // reader that sees word[layer] == value and then acquires, or starts a
@@ -96,29 +96,21 @@ __device__ __forceinline__ void write_marks(const SignalTargets& t, uint32_t lay
   }
 }
 
-// 16 bytes as two agent-coherent (write-through) 8-byte stores.
-__device__ __forceinline__ void store16_coherent(g_u32x4* p, u32x4 v) {
-  g_u64* q = reinterpret_cast<g_u64*>(p);
-  __hip_atomic_store(q, static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32),
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(q + 1, static_cast<uint64_t>(v.z) | (static_cast<uint64_t>(v.w) << 32),
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Called by one lane per workgroup once the workgroup's stores of chunk c are
-// acknowledged.  marks.chunk_start[0..n] are the launch-relative first
-// chunks of its layers (increasing, chunk_start[0] == 0 <= c <
-// chunk_start[n]); the search keeps chunk_start[lo] <= c < chunk_start[hi].
-__device__ __forceinline__ void tile_done(const LayerMarks& m, uint32_t c,
-                                          uint32_t tiles_per_chunk) {
+// acknowledged.  start[0..n] are the launch-relative first chunks of its
+// layers (increasing, start[0] == 0 <= c < start[n]; m's own table or a copy
+// of it in LDS, as layer[]); the search keeps start[lo] <= c < start[hi].
+template <class Table>
+__device__ __forceinline__ void tile_done(const LayerMarks& m, Table start, Table layers,
+                                          uint32_t c, uint32_t tiles_per_chunk) {
   uint32_t lo = 0, hi = m.n;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (m.chunk_start[mid] <= c) lo = mid;
+    if (start[mid] <= c) lo = mid;
     else hi = mid;
   }
-  const uint32_t layer = m.layer[lo];
-  const uint32_t tiles = (m.chunk_start[lo + 1] - m.chunk_start[lo]) * tiles_per_chunk;
+  const uint32_t layer = layers[lo];
+  const uint32_t tiles = (start[lo + 1] - start[lo]) * tiles_per_chunk;
   uint32_t* cnt = m.counters + layer * kCounterStride;
   const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
@@ -160,6 +152,13 @@ __device__ __forceinline__ MarkGroup mark_group(const SliceMarks& m, uint32_t wg
       g = {m.wg_start[i], m.chunk_start[i], m.chunk_start[i + 1] - m.chunk_start[i], m.units[i],
            m.layer[i]};
   return g;
+}
+
+// A value that every lane of the wave holds, in scalar registers.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
 // 16 bytes at base + 16 * lane, written through the XCD's L2 to the device's
@@ -321,25 +320,58 @@ copy_chunks_v16_kernel(const ChunkDesc* __restrict__ descs, uint32_t units_per_c
 // pull, so it puts both words back to 0.  The launch therefore leaves the
 // queue as it found it, whatever the host knows of earlier launches: a
 // replayed graph or a launch on another stream after this one finds 0.
-// Launches that run at the same time need queues of their own.  MARK adds
-// the per-layer completion marks, with agent-coherent stores (see
+// Launches that run at the same time need queues of their own.
+//
+// A small call's descriptors lie in pinned host memory: reading one in front of
+// each tile put a host-link round trip there, 2 us idle and as long as the
+// posted writes ahead of it take in a save.  Each workgroup takes the whole
+// table (at most kQueueTableMax descriptors, and the layers' table of a marking
+// launch) into LDS first (kQueueTable): 64 chunks of 32 KiB load in 73.5 ->
+// 67.6 us, 320 in 226 -> 213 (call and wait; the link takes 36.6 and 183, an
+// empty kernel and its wait 9.5).  A pull waits for its wave's stores too, and
+// those into host memory are acknowledged late, so a small save takes its tiles
+// by a fixed map instead (kFixedTable; every workgroup starts at once, and a
+// save has no layer to land first): 64 chunks save in 70.9 -> 65.6 us, 320 in
+// 252 -> 218 (with streaming stores and 8 workgroups, PF_SAVE_HOST_DEFAULT_*).
+// Fetching the next tile and its descriptor during the copy of this one, by a
+// wave of its own, made large copies 1-8% slower: the link runs best with few
+// requests.
+//
+// MARK adds the per-layer completion marks, with write-through stores (see
 // write_marks).
-template <int UNROLL, bool NTL, bool NTS, bool MARK>
+template <int UNROLL, bool NTL, bool NTS, bool MARK, QueueTiles TILES>
 __global__ void __launch_bounds__(1024)
-copy_chunks_queue_kernel(const ChunkDesc* __restrict__ descs, uint32_t tiles_per_chunk,
-                         uint32_t n_tiles, uint32_t chunk16, LayerMarks marks,
-                         uint32_t* queue) {
+copy_chunks_queue_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
+                         uint32_t tiles_per_chunk, uint32_t n_tiles, uint32_t chunk16,
+                         LayerMarks marks, uint32_t* queue) {
+  constexpr bool TABLE = TILES != QueueTiles::kQueue;
   __shared__ uint32_t s_tile;
+  __shared__ ChunkDesc s_desc[TABLE ? kQueueTableMax : 1];
+  __shared__ uint32_t s_start[TABLE && MARK ? kQueueTableMax + 1 : 1];
+  __shared__ uint32_t s_layer[TABLE && MARK ? kQueueTableMax : 1];
   const uint32_t stride = blockDim.x;
   const uint32_t tile_elems = stride * UNROLL;
-  for (;;) {
-    if (threadIdx.x == 0)
-      s_tile = __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const uint32_t t = s_tile;
-    __syncthreads();  // every lane has read s_tile before it is written again
+  const uint32_t lane = threadIdx.x & 63u;
+  if constexpr (TABLE) {
+    // Read by every lane after the next barrier.
+    for (uint32_t i = threadIdx.x; i < n_chunks; i += stride) s_desc[i] = descs[i];
+    if constexpr (MARK) {
+      for (uint32_t i = threadIdx.x; i <= marks.n; i += stride) s_start[i] = marks.chunk_start[i];
+      for (uint32_t i = threadIdx.x; i < marks.n; i += stride) s_layer[i] = marks.layer[i];
+    }
+  }
+  if constexpr (TILES == QueueTiles::kFixedTable) __syncthreads();
+  for (uint32_t fixed = blockIdx.x;; fixed += gridDim.x) {
+    uint32_t t = fixed;
+    if constexpr (TILES != QueueTiles::kFixedTable) {
+      if (threadIdx.x == 0)
+        s_tile = __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      t = s_tile;
+      __syncthreads();  // every lane has read s_tile before it is written again
+    }
     if (t >= n_tiles) {  // uniform: the queue is empty for every later pull too
-      if (threadIdx.x == 0) {
+      if (TILES != QueueTiles::kFixedTable && threadIdx.x == 0) {
         const uint32_t out = __hip_atomic_fetch_add(queue + 1, 1u, __ATOMIC_ACQ_REL,
                                                     __HIP_MEMORY_SCOPE_AGENT);
         if (out + 1 == gridDim.x) {
@@ -351,20 +383,25 @@ copy_chunks_queue_kernel(const ChunkDesc* __restrict__ descs, uint32_t tiles_per
     }
     const uint32_t c = t / tiles_per_chunk;
     const uint32_t tile = t - c * tiles_per_chunk;
-    const ChunkDesc d = descs[c];
+    const ChunkDesc d = TABLE ? s_desc[c] : descs[c];
     const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src);
     g_u32x4* __restrict__ dst = reinterpret_cast<g_u32x4*>(d.dst);
     const uint32_t tile_base = tile * tile_elems;
     const uint32_t base_e = tile_base + threadIdx.x;
+    auto put = [&](uint32_t e, u32x4 v) {  // word e, of this lane
+      if constexpr (MARK)
+        store16_through(uniform64(d.dst) +
+                            static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(e - lane)) * 16u,
+                        1024u, lane, v);
+      else
+        store16<NTS>(dst + e, v);
+    };
     u32x4 v[UNROLL];
     if (tile_base + tile_elems <= chunk16) {
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) v[u] = load16<NTL>(src + base_e + u * stride);
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if constexpr (MARK) store16_coherent(dst + base_e + u * stride, v[u]);
-        else store16<NTS>(dst + base_e + u * stride, v[u]);
-      }
+      for (int u = 0; u < UNROLL; ++u) put(base_e + u * stride, v[u]);
     } else {
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
@@ -374,16 +411,18 @@ copy_chunks_queue_kernel(const ChunkDesc* __restrict__ descs, uint32_t tiles_per
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
         const uint32_t e = base_e + u * stride;
-        if (e < chunk16) {
-          if constexpr (MARK) store16_coherent(dst + e, v[u]);
-          else store16<NTS>(dst + e, v[u]);
-        }
+        if (e < chunk16) put(e, v[u]);
       }
     }
     if constexpr (MARK) {
       __builtin_amdgcn_s_waitcnt(0);  // every store of this wave acknowledged
       __syncthreads();
-      if (threadIdx.x == 0) tile_done(marks, c, tiles_per_chunk);
+      if (threadIdx.x == 0) {
+        if constexpr (TABLE)
+          tile_done(marks, s_start, s_layer, c, tiles_per_chunk);
+        else
+          tile_done(marks, marks.chunk_start, marks.layer, c, tiles_per_chunk);
+      }
     }
   }
 }
@@ -464,39 +503,42 @@ static hipError_t launch_v16(const ChunkDesc* d_descs, uint32_t units_per_chunk,
   return hipGetLastError();
 }
 
+// One queued launch.
+struct QueueLaunch {
+  dim3 grid, block;
+  hipStream_t stream;
+  const ChunkDesc* descs;
+  uint32_t n_chunks, tiles_per_chunk, n_tiles, chunk16;
+  const LayerMarks* marks;
+  uint32_t* queue;
+  QueueTiles tiles;
+};
+
+template <int UNROLL, bool NTL, bool NTS, bool MARK, QueueTiles TILES>
+static void launch_queue_as(const QueueLaunch& q) {
+  hipLaunchKernelGGL((copy_chunks_queue_kernel<UNROLL, NTL, NTS, MARK, TILES>), q.grid, q.block,
+                     0, q.stream, q.descs, q.n_chunks, q.tiles_per_chunk, q.n_tiles, q.chunk16,
+                     q.marks ? *q.marks : LayerMarks{}, q.queue);
+}
+
+// A marking launch's stores are written through, whatever the flags.
 template <int UNROLL, bool NTL, bool NTS>
-static void launch_queue_nt(dim3 grid, dim3 block, hipStream_t stream, const ChunkDesc* d,
-                            uint32_t tpc, uint32_t n_tiles, uint32_t c16,
-                            const LayerMarks* marks, uint32_t* queue) {
-  if (marks)
-    hipLaunchKernelGGL((copy_chunks_queue_kernel<UNROLL, NTL, NTS, true>), grid, block, 0,
-                       stream, d, tpc, n_tiles, c16, *marks, queue);
-  else
-    hipLaunchKernelGGL((copy_chunks_queue_kernel<UNROLL, NTL, NTS, false>), grid, block, 0,
-                       stream, d, tpc, n_tiles, c16, LayerMarks{}, queue);
+static void launch_queue_nt(const QueueLaunch& q) {
+  constexpr QueueTiles kQueue = QueueTiles::kQueue, kTable = QueueTiles::kQueueTable;
+  if (q.marks && q.tiles == kQueue) launch_queue_as<UNROLL, NTL, false, true, kQueue>(q);
+  else if (q.marks) launch_queue_as<UNROLL, NTL, false, true, kTable>(q);
+  else if (q.tiles == kQueue) launch_queue_as<UNROLL, NTL, NTS, false, kQueue>(q);
+  else if (q.tiles == kTable) launch_queue_as<UNROLL, NTL, NTS, false, kTable>(q);
+  else launch_queue_as<UNROLL, NTL, NTS, false, QueueTiles::kFixedTable>(q);
 }
 
 template <int UNROLL>
-static void launch_queue(dim3 grid, dim3 block, hipStream_t stream, const ChunkDesc* d,
-                         uint32_t tpc, uint32_t n_tiles, uint32_t c16, uint32_t flags,
-                         const LayerMarks* marks, uint32_t* queue) {
+static void launch_queue(const QueueLaunch& q, uint32_t flags) {
   switch (flags & PF_KERNEL_NONTEMPORAL) {
-    case 0:
-      launch_queue_nt<UNROLL, false, false>(grid, block, stream, d, tpc, n_tiles, c16, marks,
-                                            queue);
-      break;
-    case PF_KERNEL_NT_LOADS:
-      launch_queue_nt<UNROLL, true, false>(grid, block, stream, d, tpc, n_tiles, c16, marks,
-                                           queue);
-      break;
-    case PF_KERNEL_NT_STORES:
-      launch_queue_nt<UNROLL, false, true>(grid, block, stream, d, tpc, n_tiles, c16, marks,
-                                           queue);
-      break;
-    default:
-      launch_queue_nt<UNROLL, true, true>(grid, block, stream, d, tpc, n_tiles, c16, marks,
-                                          queue);
-      break;
+    case 0: launch_queue_nt<UNROLL, false, false>(q); break;
+    case PF_KERNEL_NT_LOADS: launch_queue_nt<UNROLL, true, false>(q); break;
+    case PF_KERNEL_NT_STORES: launch_queue_nt<UNROLL, false, true>(q); break;
+    default: launch_queue_nt<UNROLL, true, true>(q); break;
   }
 }
 
@@ -555,32 +597,36 @@ hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
 
 hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
-                                    uint32_t grid, const LayerMarks* marks,
-                                    uint32_t* queue, uint32_t* n_tiles, hipStream_t stream) {
-  *n_tiles = 0;
+                                    uint32_t grid, QueueTiles tiles, const LayerMarks* marks,
+                                    uint32_t* queue, hipStream_t stream) {
   if (n_chunks == 0 || chunk_bytes == 0) return hipSuccess;
   if (threads == 0 || threads > 1024 || threads % 64 != 0 || grid == 0 || !queue)
     return hipErrorInvalidValue;
+  // Every layer of a marking launch has a chunk, so its table fits too.
+  if (tiles != QueueTiles::kQueue &&
+      (n_chunks > kQueueTableMax || (marks && marks->n > n_chunks)))
+    return hipErrorInvalidValue;
+  if (tiles == QueueTiles::kFixedTable && marks) return hipErrorInvalidValue;
   if (marks && (marks->n == 0 || !marks->chunk_start || !marks->layer || !marks->counters ||
                 marks->targets.count == 0 || marks->targets.count > kMaxSignalTargets))
     return hipErrorInvalidValue;
   const uint32_t flags = unroll & PF_KERNEL_NONTEMPORAL;
   unroll &= 0xffu;
-  uint32_t tpc = 0, ntiles = 0, c16 = 0;
-  if (!tile_geometry(n_chunks, chunk_bytes, threads, unroll, &tpc, &ntiles, &c16))
+  QueueLaunch q{dim3(grid), dim3(threads), stream, d_descs, n_chunks, 0, 0, 0, marks, queue,
+                tiles};
+  if (!tile_geometry(n_chunks, chunk_bytes, threads, unroll, &q.tiles_per_chunk, &q.n_tiles,
+                     &q.chunk16))
     return hipErrorInvalidValue;
-  if (static_cast<uint64_t>(ntiles) + grid > 0xffffffffull) return hipErrorInvalidValue;
+  if (static_cast<uint64_t>(q.n_tiles) + grid > 0xffffffffull) return hipErrorInvalidValue;
   if (grid > kMaxGrid) return hipErrorInvalidValue;
-  const dim3 g(grid), b(threads);
   switch (unroll) {
-    case 1: launch_queue<1>(g, b, stream, d_descs, tpc, ntiles, c16, flags, marks, queue); break;
-    case 2: launch_queue<2>(g, b, stream, d_descs, tpc, ntiles, c16, flags, marks, queue); break;
-    case 4: launch_queue<4>(g, b, stream, d_descs, tpc, ntiles, c16, flags, marks, queue); break;
-    case 8: launch_queue<8>(g, b, stream, d_descs, tpc, ntiles, c16, flags, marks, queue); break;
-    case 16: launch_queue<16>(g, b, stream, d_descs, tpc, ntiles, c16, flags, marks, queue); break;
+    case 1: launch_queue<1>(q, flags); break;
+    case 2: launch_queue<2>(q, flags); break;
+    case 4: launch_queue<4>(q, flags); break;
+    case 8: launch_queue<8>(q, flags); break;
+    case 16: launch_queue<16>(q, flags); break;
     default: return hipErrorInvalidValue;
   }
-  *n_tiles = ntiles;
   return hipGetLastError();
 }
 

@@ -347,8 +347,7 @@ struct pf_xfer {
   // Launch shapes per route (PF_ROUTE_*), the fastest measured on MI355X:
   //   gather into HBM:   one streaming 16 B load per lane, round-robin order;
   //   scatter:           chosen between kScatterShapes;
-  //   save to the host:  512 threads, two streaming loads per lane, ordinary
-  //                      stores into host memory.
+  //   save to the host:  512 threads, two streaming loads and stores per lane.
   uint32_t threads[4] = {PF_SAVE_DEFAULT_THREADS, PF_LOAD_DEFAULT_THREADS,
                          PF_SAVE_HOST_DEFAULT_THREADS, PF_LOAD_HOST_DEFAULT_THREADS};
   uint32_t unroll[4] = {PF_SAVE_DEFAULT_UNROLL, PF_LOAD_DEFAULT_UNROLL,
@@ -455,10 +454,11 @@ int upload_desc(pf_xfer* x, size_t n, size_t off = 0) {
 // Small calls: a separate copy of the descriptors costs about 12 us before
 // the first kernel can start, more than the kernels of a one-block load
 // take.  Up to this many descriptors the kernels read them in place from
-// coherent pinned memory (one 16-byte read over the host link per
-// workgroup); larger calls upload them, since an HBM-bound launch would feel
-// that read in every workgroup.
-constexpr size_t kHostDescMax = 512;
+// coherent pinned memory (a queued launch's workgroups take them all into LDS,
+// a fixed-map wave reads its own); larger calls upload them, since an
+// HBM-bound launch would feel that read in every workgroup.
+constexpr size_t kHostDescMax = kQueueTableMax;
+constexpr uint32_t kInPlaceGrid = 16;
 
 // The in-place buffer for a call of n descriptors, or null when the call
 // must upload (too many, or the previous in-place call may still be read).
@@ -477,15 +477,20 @@ ChunkDesc* small_desc(pf_xfer* x, size_t n) {
 // One gather/scatter launch of the n chunks at descs on `stream`.  With
 // qgrid > 0 (16-byte aligned chunks only) it runs queued: qgrid persistent
 // workgroups pull tiles from the queue at `queue`, which no launch that may
-// overlap this one uses.  Otherwise one workgroup per tile (at most max_grid
-// workgroups, 0 = no cap).
+// overlap this one uses; `tiles` says where its descriptors lie.
+// Otherwise one workgroup per tile (at most max_grid workgroups, 0 = no cap).
 hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint64_t chunk_bytes,
                       bool al16, uint32_t threads, uint32_t unroll, uint32_t qgrid,
-                      uint32_t max_grid, const LayerMarks* marks, uint32_t* queue) {
+                      uint32_t max_grid, QueueTiles tiles, const LayerMarks* marks,
+                      uint32_t* queue) {
   (void)hipGetLastError();
   if (!(al16 && qgrid > 0))
     return launch_copy_chunks(descs, static_cast<uint32_t>(n), chunk_bytes, al16, threads, unroll,
                               max_grid, stream);
+  // Each workgroup reads the whole table of an in-place call, and few keep the
+  // link busy for it.
+  if (tiles != QueueTiles::kQueue) qgrid = std::min(qgrid, kInPlaceGrid);
+  if (max_grid && qgrid > max_grid) qgrid = max_grid;
   // Chunks smaller than a tile (e.g. 4 KiB segments of one tensor-parallel
   // rank) get workgroups sized to the chunk, and proportionally more of
   // them, so each pull moves a whole chunk with every lane busy and the
@@ -500,9 +505,8 @@ hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint
     if (max_grid && qgrid > max_grid) qgrid = max_grid;
     threads = t2;
   }
-  uint32_t n_tiles = 0;
   return launch_copy_chunks_queue(descs, static_cast<uint32_t>(n), chunk_bytes, threads, unroll,
-                                  qgrid, marks, queue, &n_tiles, stream);
+                                  qgrid, tiles, marks, queue, stream);
 }
 
 // Reads back finished scatter trials; once every candidate has been timed
@@ -600,8 +604,12 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
     if (trial) PF_HIP(hipEventRecord(trial->start, stream));
   }
   unroll &= ~PF_KERNEL_AUTO;
+  QueueTiles tiles = QueueTiles::kQueue;
+  if (x->desc_base == x->h_small)
+    tiles = dir == PF_ROUTE_SAVE_HOST && !marks ? QueueTiles::kFixedTable : QueueTiles::kQueueTable;
   const hipError_t e = issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16,
-                                  threads, unroll, qgrid, x->max_grid, marks, queue);
+                                  threads, unroll, qgrid, x->max_grid,
+                                  tiles, marks, queue);
   if (e != hipSuccess) return hip_fail(e, "gather/scatter kernel launch");
   if (trial) {
     PF_HIP(hipEventRecord(trial->stop, stream));
@@ -2133,7 +2141,7 @@ int pf_load_layers_noalloc(pf_stream stream, const pf_layer_xfer* layers, uint32
           s, d_desc + first, n, p.chunk_bytes, al,
           host ? PF_LOAD_HOST_DEFAULT_THREADS : PF_LOAD_DEFAULT_THREADS,
           host ? PF_LOAD_HOST_DEFAULT_UNROLL : (PF_LOAD_DEFAULT_UNROLL & ~PF_KERNEL_AUTO),
-          host ? PF_LOAD_HOST_DEFAULT_GRID : 0, 0, nullptr, queue);
+          host ? PF_LOAD_HOST_DEFAULT_GRID : 0, 0, QueueTiles::kQueue, nullptr, queue);
       if (e != hipSuccess) return hip_fail(e, "gather/scatter kernel launch");
       first += n;
       li = lj;

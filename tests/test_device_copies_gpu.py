@@ -1,9 +1,11 @@
-"""GPU tests of copies between device buffers at the edges of the kernels' tiles.
+"""GPU tests of the copy kernels at the edges of their tiles.
 
 A kernel-mode save into, or load out of, a buffer in device memory moves each
-chunk as units of one wave.  The sizes here sit at the edges of a unit (one
-wave's words, one more, one less), of a workgroup's share and of a launch.  The
-expected bytes are a numpy indexing of the same layout.
+chunk as units of one wave; one that crosses the host link takes tiles from a
+queue, or by a fixed map.  The sizes here sit at the edges of a unit or a tile
+(one wave's words, one more, one less), of a workgroup's share, of the
+descriptor table that small calls read in place, and of a launch.  The expected
+bytes are a numpy indexing of the same layout.
 """
 
 import numpy as np
@@ -122,4 +124,42 @@ def test_fixed_map_copies(gpu, bpb, segs, n):
         ctx.load_layers([layer.transfer(pool.ptr)], _lib.MODE_KERNEL)
         ctx.synchronize()
         assert np.array_equal(layer.dev.download(), layer.host), f"scatter {threads} {unroll:#x}"
+    ctx.close()
+
+
+# Launches of one chunk, of the largest descriptor table read in place and of one
+# chunk more, over one layer and over many; whole, partial and tiny tiles.
+SMALL = [(bpb, segs, counts) for bpb in (16, 1040, 16400)
+         for segs, counts in ((1, (1,)), (2, (3, 0, 1, 4)), (1, (510, 0, 2)), (1, (511, 2)),
+                              (2, (1,) * 256))]
+
+
+@pytest.mark.parametrize("bpb,segs,counts", SMALL)
+def test_small_host_copies(gpu, bpb, segs, counts):
+    """Zero-copy save, load and marked load of few chunks, with one workgroup, a few,
+    and more than there are tiles."""
+    rng = np.random.default_rng(bpb + len(counts))
+    layers = make_layers(rng, bpb, segs, counts, max(counts) + 3)
+    pool = PinnedBuffer(sum(l.nbytes for l in layers))
+    words = PinnedBuffer(8 * len(layers))
+    words.array[:] = 0
+    ctx = TransferContext(0)
+    xfers = [l.transfer(b) for l, b in zip(layers, bases(layers, pool.ptr))]
+    for value, grid in ((1, 1), (2, 3), (3, 64)):
+        for route in (_lib.ROUTE_SAVE_HOST, _lib.ROUTE_LOAD_HOST):
+            ctx.set_route_grid(route, grid)
+        pool.array[:] = 0
+        ctx.save_layers(xfers, _lib.MODE_KERNEL)
+        assert np.array_equal(pool.array, np.concatenate([l.packed() for l in layers]))
+        for marked in (False, True):
+            pool.array[:] = rng.integers(0, 256, pool.nbytes, np.uint8)
+            if marked:
+                ctx.load_layers_marked(xfers, [(words.ptr, value, True)], _lib.MODE_KERNEL)
+            else:
+                ctx.load_layers(xfers, _lib.MODE_KERNEL)
+            ctx.synchronize()
+            for l, at in zip(layers, bases(layers, 0)):
+                l.restore(pool.array[at:at + l.nbytes])
+                assert np.array_equal(l.dev.download(), l.host)
+        assert words.array.view(np.uint64).tolist() == [value] * len(layers)
     ctx.close()
