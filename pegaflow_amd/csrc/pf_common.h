@@ -128,9 +128,10 @@ struct LayerList {
   uint32_t ids[kLayerListMax];
 };
 
-// Kernel launchers (pf_kernels.hip).
+// Kernel launchers (pf_kernels.hip).  host_side: the far side of the copy is
+// host memory.
 hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
-                              uint64_t chunk_bytes, bool aligned16,
+                              uint64_t chunk_bytes, bool aligned16, bool host_side,
                               uint32_t threads, uint32_t unroll,
                               uint32_t max_grid, hipStream_t stream);
 // The queued copy (16-byte aligned chunks only): `grid` persistent

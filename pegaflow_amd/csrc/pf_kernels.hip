@@ -29,6 +29,8 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // Global-address-space views: the addresses arrive as integers, and without
 // the address space the compiler would emit generic (flat) accesses.
 typedef __attribute__((address_space(1))) u32x4 g_u32x4;
+typedef u32x4 u32x4_any __attribute__((aligned(1)));  // at any address
+typedef __attribute__((address_space(1))) u32x4_any g_u32x4_any;
 typedef __attribute__((address_space(1))) uint8_t g_u8;
 typedef __attribute__((address_space(1))) uint64_t g_u64;
 
@@ -451,7 +453,10 @@ __global__ void wait_word_kernel(const uint64_t* word, uint64_t value, uint64_t 
   }
 }
 
-// Fallback for chunks whose addresses or size are not 16-byte aligned.
+// Chunks whose addresses or size are not 16-byte aligned, over the host link: a
+// byte per lane.  The link is the bound: 59 MB in 12,300-byte chunks load in
+// 1,095-1,186 us and save in 1,100, where the link takes 1,032 (by 16-byte words,
+// as below, 1,072 and 1,108-1,145).
 __global__ void __launch_bounds__(1024)
 copy_chunks_b1_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
                       uint64_t chunk_bytes) {
@@ -460,6 +465,44 @@ copy_chunks_b1_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
     const g_u8* __restrict__ src = reinterpret_cast<const g_u8*>(d.src);
     g_u8* __restrict__ dst = reinterpret_cast<g_u8*>(d.dst);
     for (uint64_t i = threadIdx.x; i < chunk_bytes; i += blockDim.x) dst[i] = src[i];
+  }
+}
+
+// The same between device buffers, by units as in the fixed map.  A chunk's
+// stores are 16-byte words at aligned addresses, its loads the 16 bytes that go
+// there, at whatever address they have; up to 15 bytes in front of the first
+// word go with the chunk's first unit and those behind the last word with its
+// last.  Bound by HBM: 59 MB in 12,300-byte chunks take 27 us, byte by byte 61;
+// 200-byte chunks 66 and 115.  (Aligned loads shifted between the lanes were no
+// faster.)
+__global__ void __launch_bounds__(kFixedThreads)
+copy_chunks_unaligned_kernel(const ChunkDesc* __restrict__ descs, uint32_t units_per_chunk,
+                             uint32_t n_units, uint64_t chunk_bytes) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t waves = blockDim.x >> 6;
+  const uint32_t n_wg = (n_units + waves - 1) / waves;
+  for (uint32_t b = blockIdx.x; b < n_wg; b += gridDim.x) {
+    const uint32_t unit =
+        __builtin_amdgcn_readfirstlane(b * waves + (threadIdx.x >> 6));
+    if (unit >= n_units) continue;
+    const uint32_t c = unit / units_per_chunk;
+    const uint32_t u = unit - c * units_per_chunk;
+    const ChunkDesc d = descs[c];
+    const uint64_t to_word = (16u - (d.dst & 15u)) & 15u;
+    const uint64_t head = to_word < chunk_bytes ? to_word : chunk_bytes;
+    const uint64_t words = (chunk_bytes - head) >> 4;  // <= 64 * units_per_chunk
+    const uint32_t tail = static_cast<uint32_t>(chunk_bytes - head) & 15u;
+    const uint64_t src = d.src + head, dst = d.dst + head;
+    const uint64_t e0 = static_cast<uint64_t>(u) * 64u;
+    if (e0 + lane < words)
+      store16_through(dst + e0 * 16u, 1024u, lane,
+                      __builtin_nontemporal_load(
+                          reinterpret_cast<const g_u32x4_any*>(src) + e0 + lane));
+    if (u == 0 && lane < head)
+      reinterpret_cast<g_u8*>(d.dst)[lane] = reinterpret_cast<const g_u8*>(d.src)[lane];
+    if (u == units_per_chunk - 1 && lane < tail)
+      reinterpret_cast<g_u8*>(dst + words * 16u)[lane] =
+          reinterpret_cast<const g_u8*>(src + words * 16u)[lane];
   }
 }
 
@@ -565,7 +608,7 @@ static bool tile_geometry(uint32_t n_chunks, uint64_t chunk_bytes, uint32_t thre
 // `unroll` carries the loads in flight per lane (low byte) and the
 // PF_KERNEL_NT_LOADS / PF_KERNEL_NT_STORES / PF_KERNEL_XCD_MAJOR flags.
 hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
-                              uint64_t chunk_bytes, bool aligned16,
+                              uint64_t chunk_bytes, bool aligned16, bool host_side,
                               uint32_t threads, uint32_t unroll,
                               uint32_t max_grid, hipStream_t stream) {
   if (n_chunks == 0 || chunk_bytes == 0) return hipSuccess;
@@ -573,6 +616,19 @@ hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
   const uint32_t flags = unroll & (PF_KERNEL_NONTEMPORAL | PF_KERNEL_XCD_MAJOR);
   unroll &= 0xffu;
   if (max_grid > kMaxGrid) max_grid = kMaxGrid;
+  if (!aligned16 && !host_side) {
+    uint64_t upc = (chunk_bytes / 16 + 63) / 64;
+    if (upc == 0) upc = 1;
+    const uint64_t units = upc * n_chunks;
+    if (units > 0xffffffffu - 16u) return hipErrorInvalidValue;
+    const uint32_t waves = kFixedThreads / 64;
+    const uint32_t n_wg = static_cast<uint32_t>((units + waves - 1) / waves);
+    const uint32_t cap = max_grid ? max_grid : kMaxGrid;
+    hipLaunchKernelGGL(copy_chunks_unaligned_kernel, dim3(n_wg < cap ? n_wg : cap),
+                       dim3(kFixedThreads), 0, stream, d_descs, static_cast<uint32_t>(upc),
+                       static_cast<uint32_t>(units), chunk_bytes);
+    return hipGetLastError();
+  }
   if (!aligned16) {
     const uint32_t grid = n_chunks < kMaxGrid ? n_chunks : kMaxGrid;
     hipLaunchKernelGGL(copy_chunks_b1_kernel, dim3(grid), dim3(threads), 0,

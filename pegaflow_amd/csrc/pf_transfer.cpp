@@ -442,7 +442,7 @@ int upload_desc(pf_xfer* x, size_t n, size_t off = 0) {
   *boot = ChunkDesc{reinterpret_cast<uint64_t>(x->h_desc + off),
                     reinterpret_cast<uint64_t>(x->d_desc + off)};
   (void)hipGetLastError();
-  const hipError_t e = launch_copy_chunks(boot, 1, n * sizeof(ChunkDesc), true,
+  const hipError_t e = launch_copy_chunks(boot, 1, n * sizeof(ChunkDesc), true, true,
                                           kDescUploadThreads, 1, 0, s);
   if (e != hipSuccess) return hip_fail(e, "descriptor upload kernel launch");
   PF_HIP(hipEventRecord(x->desc_uploaded, s));
@@ -480,13 +480,13 @@ ChunkDesc* small_desc(pf_xfer* x, size_t n) {
 // overlap this one uses; `tiles` says where its descriptors lie.
 // Otherwise one workgroup per tile (at most max_grid workgroups, 0 = no cap).
 hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint64_t chunk_bytes,
-                      bool al16, uint32_t threads, uint32_t unroll, uint32_t qgrid,
-                      uint32_t max_grid, QueueTiles tiles, const LayerMarks* marks,
+                      bool al16, bool host_side, uint32_t threads, uint32_t unroll,
+                      uint32_t qgrid, uint32_t max_grid, QueueTiles tiles, const LayerMarks* marks,
                       uint32_t* queue) {
   (void)hipGetLastError();
   if (!(al16 && qgrid > 0))
-    return launch_copy_chunks(descs, static_cast<uint32_t>(n), chunk_bytes, al16, threads, unroll,
-                              max_grid, stream);
+    return launch_copy_chunks(descs, static_cast<uint32_t>(n), chunk_bytes, al16, host_side,
+                              threads, unroll, max_grid, stream);
   // Each workgroup reads the whole table of an in-place call, and few keep the
   // link busy for it.
   if (tiles != QueueTiles::kQueue) qgrid = std::min(qgrid, kInPlaceGrid);
@@ -607,7 +607,7 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
   QueueTiles tiles = QueueTiles::kQueue;
   if (x->desc_base == x->h_small)
     tiles = dir == PF_ROUTE_SAVE_HOST && !marks ? QueueTiles::kFixedTable : QueueTiles::kQueueTable;
-  const hipError_t e = issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16,
+  const hipError_t e = issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16, host_side,
                                   threads, unroll, qgrid, x->max_grid,
                                   tiles, marks, queue);
   if (e != hipSuccess) return hip_fail(e, "gather/scatter kernel launch");
@@ -2138,7 +2138,7 @@ int pf_load_layers_noalloc(pf_stream stream, const pf_layer_xfer* layers, uint32
       const bool host = host_side_pinned(p);
       if (int rc = check_launch_size(n, p.chunk_bytes)) return rc;
       const hipError_t e = issue_copy(
-          s, d_desc + first, n, p.chunk_bytes, al,
+          s, d_desc + first, n, p.chunk_bytes, al, host,
           host ? PF_LOAD_HOST_DEFAULT_THREADS : PF_LOAD_DEFAULT_THREADS,
           host ? PF_LOAD_HOST_DEFAULT_UNROLL : (PF_LOAD_DEFAULT_UNROLL & ~PF_KERNEL_AUTO),
           host ? PF_LOAD_HOST_DEFAULT_GRID : 0, 0, QueueTiles::kQueue, nullptr, queue);

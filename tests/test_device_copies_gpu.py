@@ -163,3 +163,33 @@ def test_small_host_copies(gpu, bpb, segs, counts):
                 assert np.array_equal(l.dev.download(), l.host)
         assert words.array.view(np.uint64).tolist() == [value] * len(layers)
     ctx.close()
+
+
+# Chunks shorter than a word, around one, around a unit, and of several units, at
+# every kind of offset from a word's boundary.
+UNALIGNED = [(bpb, off) for bpb in (1, 7, 15, 16, 17, 33, 200, 1009, 1023, 1025, 1041, 2060, 12301)
+             for off in (0, 1, 4, 15)]
+
+
+@pytest.mark.parametrize("bpb,off", UNALIGNED)
+def test_unaligned_copies(gpu, bpb, off):
+    """Gather and scatter of chunks at odd addresses: every byte of the chunks, and none
+    beside them, with and without a capped grid."""
+    rng = np.random.default_rng(bpb * 16 + off)
+    (layer,) = make_layers(rng, bpb, 2, (23,), 40)
+    pool = DeviceBuffer((layer.nbytes + 48) // 8 * 8)
+    ctx = TransferContext(0)
+    xfer = layer.transfer(pool.ptr + off)
+    for cap in (0, 2):
+        ctx.set_max_grid(cap)
+        pool.memset(0xa5)
+        ctx.save_layers([xfer], _lib.MODE_KERNEL)
+        got = pool.download()
+        assert np.array_equal(got[off:off + layer.nbytes], layer.packed())
+        assert (got[:off] == 0xa5).all() and (got[off + layer.nbytes:] == 0xa5).all()
+        pool.fill_random(bpb + cap)
+        layer.restore(pool.download(layer.nbytes, off))
+        ctx.load_layers([xfer], _lib.MODE_KERNEL)
+        ctx.synchronize()
+        assert np.array_equal(layer.dev.download(), layer.host)
+    ctx.close()
