@@ -33,6 +33,14 @@ struct LayerPlan {
   // True when the chunks must be copied one after another in list order to
   // reproduce the reference's result (needs_order in pf_transfer.cpp).
   bool ordered = false;
+  // What the checks of a call ask about all chunks, gathered while they are
+  // listed (plan_layer): all addresses of a side OR-ed together, the lowest and
+  // highest host address, whether every host chunk begins at or past the end of
+  // the one before, and the highest block named.
+  uint64_t dev_or = 0, host_or = 0;
+  uint64_t host_lo = 0, host_hi = 0;
+  bool host_increasing = true;
+  uint64_t max_block = 0;
 };
 
 struct Piece {

@@ -38,13 +38,10 @@ bool device_chunks_disjoint(const pf_kv_layout& l) {
   return kind == PF_LAYOUT_CONTIGUOUS && l.segments <= 1;
 }
 
-// Host-side chunks are pairwise disjoint (checked in O(n) for the usual
-// increasing order, else after sorting a copy).
+// Host-side chunks are pairwise disjoint (known for the usual increasing
+// order, else checked after sorting a copy).
 bool host_chunks_disjoint(const LayerPlan& p) {
-  bool increasing = true;
-  for (size_t i = 1; i < p.chunks.size() && increasing; ++i)
-    increasing = p.chunks[i].host >= p.chunks[i - 1].host + p.chunk_bytes;
-  if (increasing) return true;
+  if (p.host_increasing) return true;
   std::vector<uint64_t> h(p.chunks.size());
   for (size_t i = 0; i < h.size(); ++i) h[i] = p.chunks[i].host;
   std::sort(h.begin(), h.end());
@@ -75,14 +72,10 @@ SegBound seg_bound(const pf_kv_layout& l, uint64_t seg, uint64_t bytes) {
   return b;
 }
 
-int plan_layer(const pf_layer_xfer& lx, bool is_save, LayerPlan* out) {
+// plan_layer's list, block by block with every check of the reference.
+int plan_checked(const pf_layer_xfer& lx, bool is_save, int kind, LayerPlan* out) {
   const pf_kv_layout& l = lx.layout;
-  if (l.bytes_per_block == 0 || l.segments == 0 || l.num_blocks == 0)
-    return fail(PF_ERR_INVALID_ARGUMENT, "invalid KV cache layout");
-  if (lx.num_blocks > 0 && !lx.blocks)
-    return fail(PF_ERR_INVALID_ARGUMENT, "null block list");
   const uint64_t seg = l.bytes_per_block;
-  const int kind = layout_kind(l);
   out->chunks.clear();
   for (uint64_t i = 0; i < lx.num_blocks; ++i) {
     if (lx.blocks[i].block_idx < 0)
@@ -164,6 +157,126 @@ int plan_layer(const pf_layer_xfer& lx, bool is_save, LayerPlan* out) {
   return PF_OK;
 }
 
+// What a plan says about all its chunks, from the chunks themselves.
+void summarize(LayerPlan* p) {
+  p->dev_or = p->host_or = p->host_lo = p->host_hi = 0;
+  p->host_increasing = true;
+  if (p->chunks.empty()) return;
+  uint64_t prev = 0;
+  p->host_lo = p->host_hi = p->chunks[0].host;
+  for (size_t i = 0; i < p->chunks.size(); ++i) {
+    const Chunk& c = p->chunks[i];
+    p->dev_or |= c.dev;
+    p->host_or |= c.host;
+    p->host_lo = std::min(p->host_lo, c.host);
+    p->host_hi = std::max(p->host_hi, c.host);
+    if (i > 0 && c.host < prev + p->chunk_bytes) p->host_increasing = false;
+    prev = c.host;
+  }
+}
+
+// One list of chunks (the K list, the V list, or whole blocks) being planned
+// in one pass: where it writes, and what it gathers for the LayerPlan.
+struct ChunkList {
+  Chunk* at;
+  uint64_t bytes;
+  uint64_t dev_or = 0, host_or = 0, lo = ~0ull, hi = 0, first = 0, prev = 0;
+  bool increasing = true;
+
+  void add(size_t i, uint64_t dev, uint64_t host) {
+    at[i] = {dev, host};
+    dev_or |= dev;
+    host_or |= host;
+    lo = host < lo ? host : lo;
+    hi = host > hi ? host : hi;
+    if (i == 0) first = host;
+    else increasing &= host >= prev + bytes;
+    prev = host;
+  }
+};
+
+void gathered(const ChunkList& a, LayerPlan* p) {
+  p->dev_or = a.dev_or;
+  p->host_or = a.host_or;
+  p->host_lo = a.lo;
+  p->host_hi = a.hi;
+  p->host_increasing = a.increasing;
+}
+
+// The usual layer in one pass over its blocks: a split layout, or whole blocks,
+// with every block in bounds and every host address given.  False when some
+// block is not: plan_layer then goes through the checks one by one for the
+// reference's error.  One pass instead of one per check, here and in the calls'
+// later checks: 40,960 chunks of a gather between device buffers, 585 -> 520 us
+// a call with the Python layer's marshalling.
+bool plan_in_bounds(const pf_layer_xfer& lx, bool split, LayerPlan* out) {
+  const pf_kv_layout& l = lx.layout;
+  const uint64_t seg = l.bytes_per_block;
+  const size_t n = static_cast<size_t>(lx.num_blocks);
+  const uint64_t bytes = split ? seg : l.block_size_bytes;
+  const SegBound k = seg_bound(l, 0, bytes >= seg ? bytes : seg);
+  const SegBound v = split ? seg_bound(l, 1, seg) : k;
+  if (n == 0 || !k.any || !v.any) return false;
+  const uint64_t max_block = std::min(k.max_block, v.max_block);
+  out->chunk_bytes = bytes;
+  out->chunks.resize(split ? 2 * n : n);
+  ChunkList kl{out->chunks.data(), bytes}, vl{out->chunks.data() + n, bytes};
+  const uint64_t v_at = l.data_ptr + v.seg_off;
+  uint64_t top = 0;
+  bool host = true;
+  if (split) {
+    for (size_t i = 0; i < n; ++i) {
+      const pf_block_xfer& b = lx.blocks[i];
+      const uint64_t block = static_cast<uint64_t>(b.block_idx);  // a negative one is past the top
+      top = block > top ? block : top;
+      host &= b.k_host != 0;
+      kl.add(i, l.data_ptr + block * seg, b.k_host);
+      vl.add(i, v_at + block * seg, b.v_host ? b.v_host : b.k_host + seg);
+    }
+  } else {
+    for (size_t i = 0; i < n; ++i) {
+      const pf_block_xfer& b = lx.blocks[i];
+      const uint64_t block = static_cast<uint64_t>(b.block_idx);
+      top = block > top ? block : top;
+      host &= b.k_host != 0;
+      kl.add(i, l.data_ptr + block * seg, b.k_host);
+    }
+  }
+  if (!host || top > max_block) return false;
+  gathered(kl, out);
+  if (split) {
+    out->dev_or |= vl.dev_or;
+    out->host_or |= vl.host_or;
+    out->host_lo = std::min(out->host_lo, vl.lo);
+    out->host_hi = std::max(out->host_hi, vl.hi);
+    out->host_increasing &= vl.increasing && vl.first >= kl.prev + bytes;
+  }
+  out->max_block = top;
+  out->list_break = n;
+  return true;
+}
+
+int plan_layer(const pf_layer_xfer& lx, bool is_save, LayerPlan* out) {
+  const pf_kv_layout& l = lx.layout;
+  if (l.bytes_per_block == 0 || l.segments == 0 || l.num_blocks == 0)
+    return fail(PF_ERR_INVALID_ARGUMENT, "invalid KV cache layout");
+  if (lx.num_blocks > 0 && !lx.blocks)
+    return fail(PF_ERR_INVALID_ARGUMENT, "null block list");
+  const int kind = layout_kind(l);
+  if ((kind == PF_LAYOUT_SPLIT || !(kind == PF_LAYOUT_STRIDED && is_save)) &&
+      plan_in_bounds(lx, kind == PF_LAYOUT_SPLIT, out))
+    return PF_OK;
+  const int rc = plan_checked(lx, is_save, kind, out);
+  if (rc == PF_OK) {
+    summarize(out);
+    out->max_block = 0;
+    for (uint64_t i = 0; i < lx.num_blocks; ++i)
+      out->max_block =
+          std::max(out->max_block, static_cast<uint64_t>(lx.blocks[i].block_idx));
+  }
+  return rc;
+}
+
 // Parallel kernels give the reference's bytes only when no two chunks write
 // the same byte.  The reference copies in list order, so for a load that
 // names a block twice the later copy wins: only the last occurrence is kept.
@@ -187,11 +300,10 @@ void apply_write_policy(const pf_layer_xfer& lx, bool is_save, bool staged, Laye
   // across layers and calls instead of a zeroed one per layer).
   thread_local std::vector<uint32_t> stamp;
   thread_local uint32_t epoch = 0;
-  for (size_t i = 0; i < n; ++i)
-    if (static_cast<uint64_t>(lx.blocks[i].block_idx) >= nb) {
-      p->ordered = true;
-      return;
-    }
+  if (p->max_block >= nb) {
+    p->ordered = true;
+    return;
+  }
   if (stamp.size() < nb) stamp.resize(static_cast<size_t>(nb), 0);
   if (++epoch == 0) {  // wrapped: clear, so no old stamp can match
     std::fill(stamp.begin(), stamp.end(), 0);
@@ -220,6 +332,7 @@ void apply_write_policy(const pf_layer_xfer& lx, bool is_save, bool staged, Laye
   }
   p->chunks.swap(kept);
   if (per_block == 1) p->list_break = p->chunks.size();
+  summarize(p);
 }
 
 // The layer tensor must lie inside one device allocation and each host-side
@@ -237,13 +350,10 @@ int check_host_chunks(RangeCache& rc, const LayerPlan& p) {
   if (p.chunks.empty()) return PF_OK;
   // The usual case: every chunk inside one allocation (the pool), checked
   // as the span from the lowest to the end of the highest.
-  uint64_t lo = p.chunks[0].host, hi = p.chunks[0].host;
-  for (const Chunk& c : p.chunks) {
-    lo = c.host < lo ? c.host : lo;
-    hi = c.host > hi ? c.host : hi;
-  }
   uint64_t end = 0;
-  if (!__builtin_add_overflow(hi, p.chunk_bytes, &end) && rc.check(lo, end - lo)) return PF_OK;
+  if (!__builtin_add_overflow(p.host_hi, p.chunk_bytes, &end) &&
+      rc.check(p.host_lo, end - p.host_lo))
+    return PF_OK;
   for (const Chunk& c : p.chunks)
     if (!rc.check(c.host, p.chunk_bytes))
       return fail(PF_ERR_INVALID_ARGUMENT,
@@ -717,10 +827,7 @@ int check_all_kernel(const pf_layer_xfer* layers, const std::vector<LayerPlan>& 
 }
 
 bool chunks_aligned(const LayerPlan& p) {
-  if (!aligned16(p.chunk_bytes)) return false;
-  for (const Chunk& c : p.chunks)
-    if (!aligned16(c.dev) || !aligned16(c.host)) return false;
-  return true;
+  return aligned16(p.chunk_bytes | p.dev_or | p.host_or);
 }
 
 // ---- DMA modes ------------------------------------------------------------
@@ -810,12 +917,7 @@ bool save_hosts_disjoint(const std::vector<LayerPlan>& plans) {
   for (const LayerPlan& p : plans) {
     if (p.chunks.empty()) continue;
     if (!host_chunks_disjoint(p)) return false;
-    uint64_t lo = p.chunks[0].host, hi = p.chunks[0].host;
-    for (const Chunk& c : p.chunks) {
-      lo = std::min(lo, c.host);
-      hi = std::max(hi, c.host);
-    }
-    spans.push_back({lo, hi + p.chunk_bytes});
+    spans.push_back({p.host_lo, p.host_hi + p.chunk_bytes});
   }
   std::sort(spans.begin(), spans.end());
   bool interleaved = false;
@@ -842,6 +944,14 @@ void for_each_step_chunk(const std::vector<LayerPlan>& plans, const StagedPlan& 
     const LayerPlan& p = plans[pc.layer];
     for (size_t i = pc.begin; i < pc.end; ++i) fn(p.chunks[i], k++);
   }
+}
+
+// Every layer of a staged step has its chunks 16-byte aligned in HBM.
+bool step_aligned(const std::vector<LayerPlan>& plans, const StagedPlan& sp,
+                  const StagedStep& st) {
+  for (size_t pi = st.piece_begin; pi < st.piece_end; ++pi)
+    if (!aligned16(plans[sp.pieces[pi].layer].dev_or)) return false;
+  return true;
 }
 
 // PEGAFLOW_TRACE: microseconds from the start of a staged call to each of
@@ -880,13 +990,9 @@ bool hosts_pinned(const std::vector<LayerPlan>& plans, uint32_t begin, uint32_t 
   for (uint32_t li = begin; li < end; ++li) {
     const LayerPlan& p = plans[li];
     if (p.chunks.empty() || p.ordered) continue;
-    uint64_t lo = p.chunks[0].host, hi = p.chunks[0].host;
-    for (const Chunk& c : p.chunks) {
-      lo = std::min(lo, c.host);
-      hi = std::max(hi, c.host);
-    }
+    const uint64_t end = p.host_hi + p.chunk_bytes;
     uint64_t b = 0, e = 0;
-    if (hi + p.chunk_bytes >= hi && pinned_lookup(lo, hi + p.chunk_bytes - lo, &b, &e)) continue;
+    if (end >= p.host_hi && pinned_lookup(p.host_lo, end - p.host_lo, &b, &e)) continue;
     for (const Chunk& c : p.chunks)
       if (!pinned_lookup(c.host, p.chunk_bytes, &b, &e)) return false;
   }
@@ -1086,16 +1192,13 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
     if (st.ordered_layer >= 0 || st.piece_end - st.piece_begin > kSliceMarkLayers ||
         !aligned16(st.chunk_bytes) || !aligned16(slot_base(slice_of[si])))
       return false;
-    bool al = true;
-    for_each_step_chunk(plans, sp, st, [&](const Chunk& c, size_t) { al = al && aligned16(c.dev); });
-    return al;
+    return step_aligned(plans, sp, st);
   };
   auto kernel = [&](size_t si) -> int {
     const StagedStep& st = sp.steps[si];
     const uint64_t slot = slot_base(slice_of[si]);
-    bool al16 = aligned16(st.chunk_bytes) && aligned16(slot);
-    for_each_step_chunk(plans, sp, st,
-                        [&](const Chunk& c, size_t) { al16 = al16 && aligned16(c.dev); });
+    const bool al16 =
+        aligned16(st.chunk_bytes) && aligned16(slot) && step_aligned(plans, sp, st);
     // A slice's scatter marks the layers it completes: beside other work
     // filling every CU, each kernel of ours waits for one of that work's
     // kernels to end, so a layer lands after one such wait instead of two (a
@@ -1460,9 +1563,7 @@ int staged(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers, bool is
     } else {
       const uint64_t slot = x->staging + static_cast<uint64_t>(L) * x->slot_bytes;
       const uint64_t cb = st.chunk_bytes;
-      bool al16 = aligned16(cb) && aligned16(slot);
-      for_each_step_chunk(plans, sp, st,
-                          [&](const Chunk& c, size_t) { al16 = al16 && aligned16(c.dev); });
+      const bool al16 = aligned16(cb) && aligned16(slot) && step_aligned(plans, sp, st);
       // The host-contiguous runs of the step, each one DMA copy to or from
       // its place in the slot.
       auto copy_runs = [&]() {
@@ -1712,8 +1813,10 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
 // takes ~0.1 ms) start with an eighth of their layers: that part's copy
 // (2.9 ms for a Llama prefix, 0.37 ms for one tensor-parallel rank's) hides
 // the planning of the rest, and one more launch boundary costs under 1%.
-// Copies between device buffers, HBM-bound at about 0.05 ms for such a
-// first part, are issued whole, as one launch.
+// A copy between device buffers, HBM-bound, starts with a quarter (about 0.11
+// ms of a Llama prefix), which hides the planning of the rest too since that
+// takes one pass: the prefix's gather took 513-525 us issued whole and 488 in
+// two parts, its scatter 555-561 and 512 (4 KiB chunks, 147 and 157, either way).
 constexpr uint64_t kPipelineMinChunks = 16384;
 
 }  // namespace
@@ -1733,8 +1836,9 @@ uint32_t pipeline_head(const pf_layer_xfer* layers, uint32_t num_layers) {
     if (!first && layers[i].num_blocks > 0 && layers[i].blocks) first = layers[i].blocks;
   }
   uint64_t b = 0, e = 0;
-  if (!first || !pinned_lookup(first->k_host, 1, &b, &e)) return 0;
-  return pipeline_head_layers(num_layers, chunks);
+  if (!first) return 0;
+  const uint32_t head = pipeline_head_layers(num_layers, chunks);
+  return head > 0 && !pinned_lookup(first->k_host, 1, &b, &e) ? num_layers / 4 : head;
 }
 
 // pending: the layers from `head` on are filled in by pending->ready(),

@@ -174,31 +174,38 @@ class LayerTransfer:
 
 
 def _layer_c(lt: LayerTransfer):
-    """The layer's pf_layer_xfer and the block array it points into, made
-    once per (registration, blocks array) pair and kept on the object: a
-    caller that passes the same layers each step (a worker's registered
-    layers) pays the marshalling once.  The array is held with the struct,
-    so the pointer stays valid; its contents may change between calls."""
-    c = lt.__dict__.get("_c")
-    if c is not None and c[0] is lt.blocks and c[1] is lt.registration:
-        return c[2], c[3]
+    """(blocks, registration, the layer's pf_layer_xfer as bytes, the block
+    array it points into), made once per (registration, blocks array) pair
+    and kept on the object: a caller that passes the same layers each step (a
+    worker's registered layers) pays the marshalling once.  The array is held
+    with the record, so the pointer stays valid; its contents may change
+    between calls."""
     b = np.ascontiguousarray(lt.blocks, dtype=BLOCK_DTYPE)
     x = LayerXfer()
     x.layout = lt.registration.to_c()
     x.blocks = b.ctypes.data if len(b) else None
     x.num_blocks = len(b)
-    lt.__dict__["_c"] = (lt.blocks, lt.registration, x, b)
-    return x, b
+    c = lt.__dict__["_c"] = (lt.blocks, lt.registration, bytes(x), b)
+    return c
 
 
 def _layer_array(layers: Sequence[LayerTransfer]):
-    arr = (LayerXfer * max(len(layers), 1))()
+    """The call's pf_layer_xfer array, and the block arrays it points into.
+    The records are joined as bytes: a ctypes element assignment per layer
+    took 33 us of a 32-layer call, this 12."""
     keep = []
-    for i, lt in enumerate(layers):
-        x, b = _layer_c(lt)
-        arr[i] = x
-        keep.append(b)
-    return arr, keep
+    records = []
+    for lt in layers:
+        c = lt.__dict__.get("_c")
+        if c is None or c[0] is not lt.blocks or c[1] is not lt.registration:
+            c = _layer_c(lt)
+        records.append(c[2])
+        keep.append(c[3])
+    n = max(len(records), 1)
+    return (LayerXfer * n).from_buffer_copy(b"".join(records) or bytes(_LAYER_BYTES)), keep
+
+
+_LAYER_BYTES = ctypes.sizeof(LayerXfer)
 
 
 def load_layers_noalloc(layers: Sequence[LayerTransfer], stream: Stream | None = None) -> None:
