@@ -82,12 +82,32 @@ __device__ __forceinline__ uint32_t tile_of(uint32_t b, uint32_t n, bool xcd_maj
 // coherence point (store16_through: the sc1 policy that agent-scope stores
 // have) and wait for every store's acknowledgement (s_waitcnt 0) before the
 // workgroup barrier; only then does one lane bump the counter (an agent-scope
-// atomic).  The finishing workgroup acquires at agent scope,
-// puts the counter back to 0 (ready for the next launch on the stream) and
-// writes the marks as release stores, at system scope for host memory.  A
-// reader that sees word[layer] == value and then acquires, or starts a
-// kernel afterwards, sees every byte of that layer.
+// atomic).  The lane whose add completes the layer therefore knows that every
+// byte of it has reached the coherence point: it puts the counter back to 0
+// (ready for the next launch on the stream) and writes the marks, at system
+// scope for host memory, with nothing left to flush or to read again.  A
+// release would write back the L2 of its own XCD, which holds none of the
+// layer's bytes, under every other workgroup's copy: with a release and an
+// acquire per layer, 61 layers of 4.7 MB took 120 us, without 94, and 32 of
+// 5.2 MB 66 and 54 (unmarked 93 and 53).  A reader that sees word[layer] ==
+// value and then acquires, or starts a kernel afterwards, sees every byte of
+// that layer.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void layer_done(const SignalTargets& t, uint32_t* counter,
+                                           uint32_t layer) {
+  // Orders the compiler and this wave's accesses; touches no cache.
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (uint32_t i = 0; i < t.count; ++i) {
+    uint64_t* w = reinterpret_cast<uint64_t*>(t.words[i]) + layer;
+    if ((t.host_mask >> i) & 1u)
+      __hip_atomic_store(w, t.value[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    else
+      __hip_atomic_store(w, t.value[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The marks of layers that earlier kernels or copies put in place.
 __device__ __forceinline__ void write_marks(const SignalTargets& t, uint32_t layer) {
   for (uint32_t i = 0; i < t.count; ++i) {
     uint64_t* w = reinterpret_cast<uint64_t*>(t.words[i]) + layer;
@@ -117,9 +137,7 @@ __device__ __forceinline__ void tile_done(const LayerMarks& m, Table start, Tabl
   const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
   if (prev + 1 == tiles) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    write_marks(m.targets, layer);
+    layer_done(m.targets, cnt, layer);
   }
 }
 
@@ -183,8 +201,8 @@ __device__ __forceinline__ void store16_through(uint64_t base, uint32_t bytes, u
 // chunk and belongs to one wave, so a chunk of any size wastes at most part of
 // its last unit.  Workgroup w copies the consecutive units of one layer that
 // its index gives it and then adds their number to the layer's counter, once:
-// adds to one counter run one after another (about 40 ns), so one per 4 KiB
-// doubled the time of the whole copy, and one per 32 KiB costs 5-25% of it.
+// adds to one counter run one after another (about 40 ns): one per 4 KiB doubled
+// the time of the whole copy, one per 32 KiB costs 0-5% of it.
 // Workgroups start in index order, so the layers land in order.
 //
 // Visibility: as in the marking protocol above, with 16-byte write-through
@@ -193,7 +211,7 @@ __device__ __forceinline__ void store16_through(uint64_t base, uint32_t bytes, u
 // before a report.  The per-workgroup release fence that this replaces allowed
 // only 128 workgroups: a 40 MiB layer took 24 us, here 17; and 61 layers of
 // 4.7 MB, one launch and one marking kernel each before, took 450 us, here
-// 120 in one launch.
+// 94 in one launch.
 template <int UNROLL, class Marks>
 __global__ void __launch_bounds__(kMarkedThreads)
 copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape,
@@ -233,11 +251,7 @@ copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape
       uint32_t* cnt = marks.counters + g.layer * kCounterStride;
       const uint32_t prev = __hip_atomic_fetch_add(cnt, mine, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT);
-      if (prev + mine == g.units) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        write_marks(marks.targets, g.layer);
-      }
+      if (prev + mine == g.units) layer_done(marks.targets, cnt, g.layer);
     }
   }
 }
