@@ -568,7 +568,7 @@ int upload_desc(pf_xfer* x, size_t n, size_t off = 0) {
 // a fixed-map wave reads its own); larger calls upload them, since an
 // HBM-bound launch would feel that read in every workgroup.
 constexpr size_t kHostDescMax = kQueueTableMax;
-constexpr uint32_t kInPlaceGrid = 16;
+constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32;
 
 // The in-place buffer for a call of n descriptors, or null when the call
 // must upload (too many, or the previous in-place call may still be read).
@@ -598,8 +598,11 @@ hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint
     return launch_copy_chunks(descs, static_cast<uint32_t>(n), chunk_bytes, al16, host_side,
                               threads, unroll, max_grid, stream);
   // Each workgroup reads the whole table of an in-place call, and few keep the
-  // link busy for it.
-  if (tiles != QueueTiles::kQueue) qgrid = std::min(qgrid, kInPlaceGrid);
+  // link busy for it, a few more where each tile is also reported: with 8, 16,
+  // 32 and 64, 64 chunks of 32 KiB load in 61.6, 61.7, 62.4 and 64.7 us, and
+  // 488 chunks of 36 KiB, marked, in 661, 374, 356 and 358.
+  if (tiles != QueueTiles::kQueue)
+    qgrid = std::min(qgrid, marks ? kInPlaceMarkGrid : kInPlaceGrid);
   if (max_grid && qgrid > max_grid) qgrid = max_grid;
   // Chunks smaller than a tile (e.g. 4 KiB segments of one tensor-parallel
   // rank) get workgroups sized to the chunk, and proportionally more of
