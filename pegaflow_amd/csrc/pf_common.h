@@ -141,7 +141,7 @@ hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
 // finished layer is marked.  Descriptors in host memory (at most
 // kQueueTableMax) are taken into LDS first: kQueueTable, or without marks
 // kFixedTable, which takes the tiles by a fixed map.
-constexpr uint32_t kQueueTableMax = 512;
+constexpr uint32_t kQueueTableMax = 1024;
 enum class QueueTiles { kQueue, kQueueTable, kFixedTable };
 hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,

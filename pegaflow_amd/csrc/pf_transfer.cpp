@@ -564,10 +564,13 @@ int upload_desc(pf_xfer* x, size_t n, size_t off = 0) {
 // Small calls: a separate copy of the descriptors costs about 12 us before
 // the first kernel can start, more than the kernels of a one-block load
 // take.  Up to this many descriptors the kernels read them in place from
-// coherent pinned memory (a queued launch's workgroups take them all into LDS,
-// a fixed-map wave reads its own); larger calls upload them, since an
-// HBM-bound launch would feel that read in every workgroup.
-constexpr size_t kHostDescMax = kQueueTableMax;
+// coherent pinned memory: a queued launch's workgroups take them all into LDS
+// (calls with such launches: up to kQueueTableMax), a fixed-map wave reads its
+// own.  Larger calls upload them, since an HBM-bound launch would feel those
+// reads.  Measured between device buffers with 32 KiB chunks, in place and
+// uploaded: 128 chunks 24.8 and 32.0 us a call, 512 29.5 and 34.4, 1,024 36.1 and
+// 40.2, 2,048 49.2 and 51.4.
+constexpr size_t kHostDescMax = 2048;
 constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32;
 
 // The in-place buffer for a call of n descriptors, or null when the call
@@ -718,7 +721,7 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
   }
   unroll &= ~PF_KERNEL_AUTO;
   QueueTiles tiles = QueueTiles::kQueue;
-  if (x->desc_base == x->h_small)
+  if (x->desc_base == x->h_small && n <= kQueueTableMax)
     tiles = dir == PF_ROUTE_SAVE_HOST && !marks ? QueueTiles::kFixedTable : QueueTiles::kQueueTable;
   const hipError_t e = issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16, host_side,
                                   threads, unroll, qgrid, x->max_grid,
@@ -1724,6 +1727,10 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
   // Counters for marks and the tile queue of queued launches.
   if (int rc = ensure_counters(x, layer_base + plans.size())) return rc;
   ChunkDesc* hd = desc_off ? nullptr : small_desc(x, total + aux_desc);
+  // Host-side launches are queued, and take the whole table into LDS.
+  if (hd && total > kQueueTableMax)
+    for (const LayerPlan& p : plans)
+      if (!p.ordered && host_side_pinned(p)) hd = nullptr;
   if (desc_off) {
     if (desc_off + total + aux_desc > x->h_cap || desc_off + total + aux_desc > x->d_cap)
       return fail(PF_ERR_INVALID_ARGUMENT, "descriptor room not reserved");

@@ -69,6 +69,8 @@ MARKED = [(bpb, 2, (3, 0, 1, 17), 40, cap)
           for bpb in (16, 1008, 1024, 1040, 2032, 2048, 2064, 8208, 36864) for cap in (0, 3)]
 # A launch large enough for the larger share of a workgroup, blocks-first and split.
 MARKED += [(32768, 2, (300, 301), 400, 0), (36864, 1, (511, 1, 512), 600, 0)]
+# More layers than a workgroup has lanes.
+MARKED += [(1040, 2, (1, 0, 3) * 180, 20, 0), (1040, 2, (1, 0, 3) * 180, 20, 5)]
 
 
 @pytest.mark.parametrize("bpb,segs,counts,nb,cap", MARKED)
@@ -102,13 +104,15 @@ def test_marked_load_from_device_memory(gpu, bpb, segs, counts, nb, cap):
 # a last unit of one word, and launches of one chunk.
 FIXED = [(bpb, segs, n) for bpb in (16, 1008, 1024, 1040, 4096, 10240, 16400) for segs, n in
          ((1, 1), (2, 37))]
+# The largest call whose descriptors are read in place, and one chunk more.
+FIXED += [(1040, 2, 1024), (1040, 1, 2049)]
 
 
 @pytest.mark.parametrize("bpb,segs,n", FIXED)
 def test_fixed_map_copies(gpu, bpb, segs, n):
     """Gather and scatter at every shape of the fixed map, capped grids included."""
     rng = np.random.default_rng(bpb + n)
-    (layer,) = make_layers(rng, bpb, segs, (n,), 64)
+    (layer,) = make_layers(rng, bpb, segs, (n,), max(64, n + 3))
     pool = DeviceBuffer(layer.nbytes)
     ctx = TransferContext(0)
     shapes = [(t, u | f) for t in (64, 512) for u in (1, 2, 4, 8, 16)
@@ -130,8 +134,8 @@ def test_fixed_map_copies(gpu, bpb, segs, n):
 # Launches of one chunk, of the largest descriptor table read in place and of one
 # chunk more, over one layer and over many; whole, partial and tiny tiles.
 SMALL = [(bpb, segs, counts) for bpb in (16, 1040, 16400)
-         for segs, counts in ((1, (1,)), (2, (3, 0, 1, 4)), (1, (510, 0, 2)), (1, (511, 2)),
-                              (2, (1,) * 256))]
+         for segs, counts in ((1, (1,)), (2, (3, 0, 1, 4)), (1, (1022, 0, 2)), (1, (1023, 2)),
+                              (2, (1,) * 300))]
 
 
 @pytest.mark.parametrize("bpb,segs,counts", SMALL)
