@@ -338,17 +338,18 @@ enum {
 };
 /* Per-route defaults (the fastest shapes measured on MI355X): HBM gathers
  * move 1 KiB a wave in round-robin order; scatters choose on evidence
- * (PF_KERNEL_AUTO); zero-copy saves 16 KiB tiles, streaming loads and stores,
- * with 8 persistent workgroups, one per XCD: against ordinary stores, which
- * gather in the L2s until they are evicted or the kernel ends, and 32
- * workgroups, 18 MiB in 32 KiB chunks 394 -> 377 us, 5 MiB in 4 KiB chunks 147
- * -> 134, 128 MiB 2,454 -> 2,426, 1.25 GiB 23,833 -> 23,727. */
+ * (PF_KERNEL_AUTO); zero-copy saves 16 KiB tiles with streaming loads and
+ * ordinary stores into host memory, and 32 workgroups.  Streaming stores from
+ * 8 are 0.5-4% faster alone (18 MiB 394 -> 377 us, 1.25 GiB 23,833 -> 23,727)
+ * but fall behind a restore that runs beside them: both at once 78 GB/s, 88
+ * with these.  Calls of few chunks stream (their descriptors are read in
+ * place). */
 #define PF_SAVE_DEFAULT_THREADS 512u
 #define PF_SAVE_DEFAULT_UNROLL (1u | PF_KERNEL_NONTEMPORAL)
 #define PF_LOAD_DEFAULT_THREADS 512u
 #define PF_LOAD_DEFAULT_UNROLL (2u | PF_KERNEL_NONTEMPORAL | PF_KERNEL_XCD_MAJOR | PF_KERNEL_AUTO)
 #define PF_SAVE_HOST_DEFAULT_THREADS 512u
-#define PF_SAVE_HOST_DEFAULT_UNROLL (2u | PF_KERNEL_NONTEMPORAL)
+#define PF_SAVE_HOST_DEFAULT_UNROLL (2u | PF_KERNEL_NT_LOADS)
 #define PF_LOAD_HOST_DEFAULT_THREADS 512u
 #define PF_LOAD_HOST_DEFAULT_UNROLL (2u | PF_KERNEL_NONTEMPORAL | PF_KERNEL_XCD_MAJOR)
 /* Shape for one route only (PF_ROUTE_*; 0 and 1 are also "saves" and
@@ -373,7 +374,7 @@ int pf_xfer_route_shape(pf_xfer* xfer, uint32_t route, uint32_t* threads,
  * caps both kinds.  Every route may run queued: the staged mode's two
  * streams each have a queue of their own, and a queued launch leaves its
  * queue empty. */
-#define PF_SAVE_HOST_DEFAULT_GRID 8u
+#define PF_SAVE_HOST_DEFAULT_GRID 32u
 #define PF_LOAD_HOST_DEFAULT_GRID 64u
 int pf_xfer_set_route_grid(pf_xfer* xfer, uint32_t route, uint32_t workgroups);
 int pf_xfer_set_kernel_shape(pf_xfer* xfer, uint32_t threads, uint32_t unroll);

@@ -84,11 +84,11 @@ KERNEL_XCD_MAJOR = 0x400
 KERNEL_AUTO = 0x800
 SAVE_DEFAULT_SHAPE = (512, 1 | KERNEL_NONTEMPORAL)
 LOAD_DEFAULT_SHAPE = (512, 2 | KERNEL_NONTEMPORAL | KERNEL_XCD_MAJOR | KERNEL_AUTO)
-SAVE_HOST_DEFAULT_SHAPE = (512, 2 | KERNEL_NONTEMPORAL)
+SAVE_HOST_DEFAULT_SHAPE = (512, 2 | KERNEL_NT_LOADS)
 LOAD_HOST_DEFAULT_SHAPE = (512, 2 | KERNEL_NONTEMPORAL | KERNEL_XCD_MAJOR)
 # Launch-shape routes (PF_ROUTE_*): direction x where the far side lives.
 ROUTE_SAVE_DEVICE, ROUTE_LOAD_DEVICE, ROUTE_SAVE_HOST, ROUTE_LOAD_HOST = 0, 1, 2, 3
-SAVE_HOST_DEFAULT_GRID, LOAD_HOST_DEFAULT_GRID = 8, 64
+SAVE_HOST_DEFAULT_GRID, LOAD_HOST_DEFAULT_GRID = 32, 64
 DEFAULT_GRIDS = {ROUTE_SAVE_DEVICE: 0, ROUTE_LOAD_DEVICE: 0,
                  ROUTE_SAVE_HOST: SAVE_HOST_DEFAULT_GRID, ROUTE_LOAD_HOST: LOAD_HOST_DEFAULT_GRID}
 DEFAULT_SHAPES = {ROUTE_SAVE_DEVICE: SAVE_DEFAULT_SHAPE, ROUTE_LOAD_DEVICE: LOAD_DEFAULT_SHAPE,

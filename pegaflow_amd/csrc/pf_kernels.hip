@@ -348,7 +348,7 @@ copy_chunks_v16_kernel(const ChunkDesc* __restrict__ descs, uint32_t units_per_c
 // those into host memory are acknowledged late, so a small save takes its tiles
 // by a fixed map instead (kFixedTable; every workgroup starts at once, and a
 // save has no layer to land first): 64 chunks save in 70.9 -> 65.6 us, 320 in
-// 252 -> 218 (with streaming stores and 8 workgroups, PF_SAVE_HOST_DEFAULT_*).
+// 252 -> 218 (with streaming stores and 8 workgroups).
 // Fetching the next tile and its descriptor during the copy of this one, by a
 // wave of its own, made large copies 1-8% slower: the link runs best with few
 // requests.

@@ -457,7 +457,8 @@ struct pf_xfer {
   // Launch shapes per route (PF_ROUTE_*), the fastest measured on MI355X:
   //   gather into HBM:   one streaming 16 B load per lane, round-robin order;
   //   scatter:           chosen between kScatterShapes;
-  //   save to the host:  512 threads, two streaming loads and stores per lane.
+  //   save to the host:  512 threads, two streaming loads per lane, ordinary
+  //                      stores into host memory.
   uint32_t threads[4] = {PF_SAVE_DEFAULT_THREADS, PF_LOAD_DEFAULT_THREADS,
                          PF_SAVE_HOST_DEFAULT_THREADS, PF_LOAD_HOST_DEFAULT_THREADS};
   uint32_t unroll[4] = {PF_SAVE_DEFAULT_UNROLL, PF_LOAD_DEFAULT_UNROLL,
@@ -571,7 +572,7 @@ int upload_desc(pf_xfer* x, size_t n, size_t off = 0) {
 // uploaded: 128 chunks 24.8 and 32.0 us a call, 512 29.5 and 34.4, 1,024 36.1 and
 // 40.2, 2,048 49.2 and 51.4.
 constexpr size_t kHostDescMax = 2048;
-constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32;
+constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32, kInPlaceSaveGrid = 8;
 
 // The in-place buffer for a call of n descriptors, or null when the call
 // must upload (too many, or the previous in-place call may still be read).
@@ -604,8 +605,14 @@ hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint
   // link busy for it, a few more where each tile is also reported: with 8, 16,
   // 32 and 64, 64 chunks of 32 KiB load in 61.6, 61.7, 62.4 and 64.7 us, and
   // 488 chunks of 36 KiB, marked, in 661, 374, 356 and 358.
-  if (tiles != QueueTiles::kQueue)
+  // A save's stores stream: ordinary ones gather in the L2s until the kernel
+  // ends (320 chunks 252 -> 218 us with the table in LDS).
+  if (tiles == QueueTiles::kFixedTable) {
+    qgrid = std::min(qgrid, kInPlaceSaveGrid);
+    unroll |= PF_KERNEL_NT_STORES;
+  } else if (tiles == QueueTiles::kQueueTable) {
     qgrid = std::min(qgrid, marks ? kInPlaceMarkGrid : kInPlaceGrid);
+  }
   if (max_grid && qgrid > max_grid) qgrid = max_grid;
   // Chunks smaller than a tile (e.g. 4 KiB segments of one tensor-parallel
   // rank) get workgroups sized to the chunk, and proportionally more of
