@@ -209,9 +209,10 @@ __device__ __forceinline__ void store16_through(uint64_t base, uint32_t bytes, u
 // stores.  They run at the rate of ordinary ones (288 MB of 36 KiB chunks 93
 // us, ordinary 97, non-temporal 105-115), so no L2 has to be written back
 // before a report.  The per-workgroup release fence that this replaces allowed
-// only 128 workgroups: a 40 MiB layer took 24 us, here 17; and 61 layers of
-// 4.7 MB, one launch and one marking kernel each before, took 450 us, here
-// 94 in one launch.
+// only 128 workgroups.  61 layers of 4.7 MB, one launch and one marking kernel
+// each before, took 450 us, here 94 in one launch.  A launch of a single 40 MiB
+// layer (a staged slice, under the next slice's copy) is bound by its 1,280 adds
+// to one counter: 28.7 us, where 128 workgroups with fences took 24.0.
 template <int UNROLL, class Marks>
 __global__ void __launch_bounds__(kMarkedThreads)
 copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape,
