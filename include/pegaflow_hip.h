@@ -342,8 +342,7 @@ enum {
  * ordinary stores into host memory, and 32 workgroups.  Streaming stores from
  * 8 are 0.5-4% faster alone (18 MiB 394 -> 377 us, 1.25 GiB 23,833 -> 23,727)
  * but fall behind a restore that runs beside them: both at once 78 GB/s, 88
- * with these.  Calls of few chunks stream (their descriptors are read in
- * place). */
+ * with these. */
 #define PF_SAVE_DEFAULT_THREADS 512u
 #define PF_SAVE_DEFAULT_UNROLL (1u | PF_KERNEL_NONTEMPORAL)
 #define PF_LOAD_DEFAULT_THREADS 512u

@@ -138,14 +138,12 @@ hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
 // workgroups pull tiles from the two-word queue at `queue` (device memory),
 // which holds 0, 0 when the launch starts and again when it ends.  Launches
 // that may run at the same time need separate queues.  With marks, each
-// finished layer is marked.  Descriptors in host memory (at most
-// kQueueTableMax) are taken into LDS first: kQueueTable, or without marks
-// kFixedTable, which takes the tiles by a fixed map.
+// finished layer is marked.  With `table` (at most kQueueTableMax chunks, their
+// descriptors in host memory) each workgroup takes the descriptors into LDS first.
 constexpr uint32_t kQueueTableMax = 1024;
-enum class QueueTiles { kQueue, kQueueTable, kFixedTable };
 hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
-                                    uint32_t grid, QueueTiles tiles, const LayerMarks* marks,
+                                    uint32_t grid, bool table, const LayerMarks* marks,
                                     uint32_t* queue, hipStream_t stream);
 // A marked copy between device buffers (16-byte aligned chunks): each finished
 // layer of the marks is marked.  At most max_grid workgroups (0: no cap).  The

@@ -341,27 +341,22 @@ copy_chunks_v16_kernel(const ChunkDesc* __restrict__ descs, uint32_t units_per_c
 //
 // A small call's descriptors lie in pinned host memory: reading one in front of
 // each tile put a host-link round trip there, 2 us idle and as long as the
-// posted writes ahead of it take in a save.  Each workgroup takes the whole
-// table (at most kQueueTableMax descriptors, and the layers' table of a marking
-// launch) into LDS first (kQueueTable): 64 chunks of 32 KiB load in 73.5 ->
-// 67.6 us, 320 in 226 -> 213 (call and wait; the link takes 36.6 and 183, an
-// empty kernel and its wait 9.5).  A pull waits for its wave's stores too, and
-// those into host memory are acknowledged late, so a small save takes its tiles
-// by a fixed map instead (kFixedTable; every workgroup starts at once, and a
-// save has no layer to land first): 64 chunks save in 70.9 -> 65.6 us, 320 in
-// 252 -> 218 (with streaming stores and 8 workgroups).
+// posted writes ahead of it take in a save.  With TABLE each workgroup takes all
+// of them (at most kQueueTableMax, and the layers' table of a marking launch)
+// into LDS first: 64 chunks of 32 KiB load in 73 -> 62 us and save in 71 -> 64,
+// 320 load in 225 -> 208 and save in 251 -> 227 (call and wait; the link takes
+// 36.6 and 183, an empty kernel and its wait 9.5).
 // Fetching the next tile and its descriptor during the copy of this one, by a
 // wave of its own, made large copies 1-8% slower: the link runs best with few
 // requests.
 //
 // MARK adds the per-layer completion marks, with write-through stores (see
-// write_marks).
-template <int UNROLL, bool NTL, bool NTS, bool MARK, QueueTiles TILES>
+// layer_done).
+template <int UNROLL, bool NTL, bool NTS, bool MARK, bool TABLE>
 __global__ void __launch_bounds__(1024)
 copy_chunks_queue_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
                          uint32_t tiles_per_chunk, uint32_t n_tiles, uint32_t chunk16,
                          LayerMarks marks, uint32_t* queue) {
-  constexpr bool TABLE = TILES != QueueTiles::kQueue;
   __shared__ uint32_t s_tile;
   __shared__ ChunkDesc s_desc[TABLE ? kQueueTableMax : 1];
   __shared__ uint32_t s_start[TABLE && MARK ? kQueueTableMax + 1 : 1];
@@ -377,18 +372,14 @@ copy_chunks_queue_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
       for (uint32_t i = threadIdx.x; i < marks.n; i += stride) s_layer[i] = marks.layer[i];
     }
   }
-  if constexpr (TILES == QueueTiles::kFixedTable) __syncthreads();
-  for (uint32_t fixed = blockIdx.x;; fixed += gridDim.x) {
-    uint32_t t = fixed;
-    if constexpr (TILES != QueueTiles::kFixedTable) {
-      if (threadIdx.x == 0)
-        s_tile = __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      t = s_tile;
-      __syncthreads();  // every lane has read s_tile before it is written again
-    }
+  for (;;) {
+    if (threadIdx.x == 0)
+      s_tile = __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const uint32_t t = s_tile;
+    __syncthreads();  // every lane has read s_tile before it is written again
     if (t >= n_tiles) {  // uniform: the queue is empty for every later pull too
-      if (TILES != QueueTiles::kFixedTable && threadIdx.x == 0) {
+      if (threadIdx.x == 0) {
         const uint32_t out = __hip_atomic_fetch_add(queue + 1, 1u, __ATOMIC_ACQ_REL,
                                                     __HIP_MEMORY_SCOPE_AGENT);
         if (out + 1 == gridDim.x) {
@@ -569,12 +560,12 @@ struct QueueLaunch {
   uint32_t n_chunks, tiles_per_chunk, n_tiles, chunk16;
   const LayerMarks* marks;
   uint32_t* queue;
-  QueueTiles tiles;
+  bool table;
 };
 
-template <int UNROLL, bool NTL, bool NTS, bool MARK, QueueTiles TILES>
+template <int UNROLL, bool NTL, bool NTS, bool MARK, bool TABLE>
 static void launch_queue_as(const QueueLaunch& q) {
-  hipLaunchKernelGGL((copy_chunks_queue_kernel<UNROLL, NTL, NTS, MARK, TILES>), q.grid, q.block,
+  hipLaunchKernelGGL((copy_chunks_queue_kernel<UNROLL, NTL, NTS, MARK, TABLE>), q.grid, q.block,
                      0, q.stream, q.descs, q.n_chunks, q.tiles_per_chunk, q.n_tiles, q.chunk16,
                      q.marks ? *q.marks : LayerMarks{}, q.queue);
 }
@@ -582,12 +573,10 @@ static void launch_queue_as(const QueueLaunch& q) {
 // A marking launch's stores are written through, whatever the flags.
 template <int UNROLL, bool NTL, bool NTS>
 static void launch_queue_nt(const QueueLaunch& q) {
-  constexpr QueueTiles kQueue = QueueTiles::kQueue, kTable = QueueTiles::kQueueTable;
-  if (q.marks && q.tiles == kQueue) launch_queue_as<UNROLL, NTL, false, true, kQueue>(q);
-  else if (q.marks) launch_queue_as<UNROLL, NTL, false, true, kTable>(q);
-  else if (q.tiles == kQueue) launch_queue_as<UNROLL, NTL, NTS, false, kQueue>(q);
-  else if (q.tiles == kTable) launch_queue_as<UNROLL, NTL, NTS, false, kTable>(q);
-  else launch_queue_as<UNROLL, NTL, NTS, false, QueueTiles::kFixedTable>(q);
+  if (q.marks && !q.table) launch_queue_as<UNROLL, NTL, false, true, false>(q);
+  else if (q.marks) launch_queue_as<UNROLL, NTL, false, true, true>(q);
+  else if (!q.table) launch_queue_as<UNROLL, NTL, NTS, false, false>(q);
+  else launch_queue_as<UNROLL, NTL, NTS, false, true>(q);
 }
 
 template <int UNROLL>
@@ -668,23 +657,21 @@ hipError_t launch_copy_chunks(const ChunkDesc* d_descs, uint32_t n_chunks,
 
 hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
-                                    uint32_t grid, QueueTiles tiles, const LayerMarks* marks,
+                                    uint32_t grid, bool table, const LayerMarks* marks,
                                     uint32_t* queue, hipStream_t stream) {
   if (n_chunks == 0 || chunk_bytes == 0) return hipSuccess;
   if (threads == 0 || threads > 1024 || threads % 64 != 0 || grid == 0 || !queue)
     return hipErrorInvalidValue;
   // Every layer of a marking launch has a chunk, so its table fits too.
-  if (tiles != QueueTiles::kQueue &&
-      (n_chunks > kQueueTableMax || (marks && marks->n > n_chunks)))
+  if (table && (n_chunks > kQueueTableMax || (marks && marks->n > n_chunks)))
     return hipErrorInvalidValue;
-  if (tiles == QueueTiles::kFixedTable && marks) return hipErrorInvalidValue;
   if (marks && (marks->n == 0 || !marks->chunk_start || !marks->layer || !marks->counters ||
                 marks->targets.count == 0 || marks->targets.count > kMaxSignalTargets))
     return hipErrorInvalidValue;
   const uint32_t flags = unroll & PF_KERNEL_NONTEMPORAL;
   unroll &= 0xffu;
   QueueLaunch q{dim3(grid), dim3(threads), stream, d_descs, n_chunks, 0, 0, 0, marks, queue,
-                tiles};
+                table};
   if (!tile_geometry(n_chunks, chunk_bytes, threads, unroll, &q.tiles_per_chunk, &q.n_tiles,
                      &q.chunk16))
     return hipErrorInvalidValue;

@@ -1,0 +1,62 @@
+// pf_launch.h — how the transfer code (pf_transfer.cpp) shapes its launches,
+// as plain functions of sizes and settings, in a header of their own so the
+// rules are tested on the host (tests/native/launch_rules_test.cpp).
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+#include "pf_common.h"
+
+namespace pf {
+
+// A queued launch: threads per workgroup, loads in flight per lane with their
+// flags, and persistent workgroups.
+struct QueueShape {
+  uint32_t threads, unroll, grid;
+};
+
+// Whether a call of n descriptors with a launch over the host link, in chunks of
+// chunk_bytes, leaves them in host memory for its workgroups to take into LDS.
+// Every workgroup reads them all, and a save of short chunks has many workgroups
+// for few bytes: 1,024 chunks of 256 B to 2 KiB save in 62-94 us in place and
+// 51-83 uploaded, of 4 KiB in 120 and 124, 256 chunks of 1 KiB in 38.6 and 39.5.
+inline bool table_in_place(size_t n, uint64_t chunk_bytes, bool is_save) {
+  return n <= kQueueTableMax && !(is_save && n > 512 && chunk_bytes < 4096);
+}
+
+// Workgroups of a small load, and of a marked one, whose descriptors are read
+// in place.
+constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32;
+
+// The queued launch of a route set to s for chunks of chunk_bytes.  `table`: its
+// workgroups take the descriptors from host memory into LDS.  max_grid caps the
+// workgroups (0: no cap).
+//
+// A save runs as its route says, however few its chunks.  A shape of their own
+// for small ones (8 workgroups, tiles by a fixed map, streaming stores) was as
+// fast alone (64, 320 and 1,024 chunks of 32 KiB in 62, 217-240 and 624 us, so
+// 64, 227 and 646) but ran at the pace of the XCD that a restore beside it left
+// the least of the link: 1.4, 4.4 and 12.1 ms beside one, so 0.35, 0.98 and 2.0.
+inline QueueShape queue_shape(QueueShape s, uint64_t chunk_bytes, bool is_save, bool table,
+                              bool marked, uint32_t max_grid) {
+  if (table && !is_save) s.grid = std::min(s.grid, marked ? kInPlaceMarkGrid : kInPlaceGrid);
+  if (max_grid && s.grid > max_grid) s.grid = max_grid;
+  // Chunks smaller than a tile (e.g. 4 KiB segments of one tensor-parallel
+  // rank) get workgroups sized to the chunk, and proportionally more of
+  // them, so each pull moves a whole chunk with every lane busy and the
+  // bytes in flight stay the same (measured: 4 KiB-segment save 53.9 ->
+  // 55.6 GB/s).
+  const uint64_t u = s.unroll & 0xffu;
+  const uint64_t want = u ? ((chunk_bytes / 16 + u - 1) / u + 63) / 64 * 64 : s.threads;
+  if (want < s.threads) {
+    const uint32_t threads = static_cast<uint32_t>(want < 64 ? 64 : want);
+    const uint64_t grid = static_cast<uint64_t>(s.grid) * s.threads / threads;
+    s.grid = static_cast<uint32_t>(std::min<uint64_t>(grid, 1u << 16));
+    if (max_grid && s.grid > max_grid) s.grid = max_grid;
+    s.threads = threads;
+  }
+  return s;
+}
+
+}  // namespace pf

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "pf_common.h"
+#include "pf_launch.h"
 #include "pf_staged.h"
 
 using namespace pf;
@@ -572,7 +573,6 @@ int upload_desc(pf_xfer* x, size_t n, size_t off = 0) {
 // uploaded: 128 chunks 24.8 and 32.0 us a call, 512 29.5 and 34.4, 1,024 36.1 and
 // 40.2, 2,048 49.2 and 51.4.
 constexpr size_t kHostDescMax = 2048;
-constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32, kInPlaceSaveGrid = 8;
 
 // The in-place buffer for a call of n descriptors, or null when the call
 // must upload (too many, or the previous in-place call may still be read).
@@ -589,47 +589,21 @@ ChunkDesc* small_desc(pf_xfer* x, size_t n) {
 }
 
 // One gather/scatter launch of the n chunks at descs on `stream`.  With
-// qgrid > 0 (16-byte aligned chunks only) it runs queued: qgrid persistent
+// s.grid > 0 (16-byte aligned chunks only) it runs queued: persistent
 // workgroups pull tiles from the queue at `queue`, which no launch that may
-// overlap this one uses; `tiles` says where its descriptors lie.
-// Otherwise one workgroup per tile (at most max_grid workgroups, 0 = no cap).
+// overlap this one uses, with their descriptors in place (`table`) or in device
+// memory.  Otherwise a fixed map hands out units (at most max_grid workgroups,
+// 0 = no cap).
 hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint64_t chunk_bytes,
-                      bool al16, bool host_side, uint32_t threads, uint32_t unroll,
-                      uint32_t qgrid, uint32_t max_grid, QueueTiles tiles, const LayerMarks* marks,
-                      uint32_t* queue) {
+                      bool al16, bool is_save, bool host_side, QueueShape s, uint32_t max_grid,
+                      bool table, const LayerMarks* marks, uint32_t* queue) {
   (void)hipGetLastError();
-  if (!(al16 && qgrid > 0))
+  if (!(al16 && s.grid > 0))
     return launch_copy_chunks(descs, static_cast<uint32_t>(n), chunk_bytes, al16, host_side,
-                              threads, unroll, max_grid, stream);
-  // Each workgroup reads the whole table of an in-place call, and few keep the
-  // link busy for it, a few more where each tile is also reported: with 8, 16,
-  // 32 and 64, 64 chunks of 32 KiB load in 61.6, 61.7, 62.4 and 64.7 us, and
-  // 488 chunks of 36 KiB, marked, in 661, 374, 356 and 358.
-  // A save's stores stream: ordinary ones gather in the L2s until the kernel
-  // ends (320 chunks 252 -> 218 us with the table in LDS).
-  if (tiles == QueueTiles::kFixedTable) {
-    qgrid = std::min(qgrid, kInPlaceSaveGrid);
-    unroll |= PF_KERNEL_NT_STORES;
-  } else if (tiles == QueueTiles::kQueueTable) {
-    qgrid = std::min(qgrid, marks ? kInPlaceMarkGrid : kInPlaceGrid);
-  }
-  if (max_grid && qgrid > max_grid) qgrid = max_grid;
-  // Chunks smaller than a tile (e.g. 4 KiB segments of one tensor-parallel
-  // rank) get workgroups sized to the chunk, and proportionally more of
-  // them, so each pull moves a whole chunk with every lane busy and the
-  // bytes in flight stay the same (measured: 4 KiB-segment save 53.9 ->
-  // 55.6 GB/s).
-  const uint64_t u = unroll & 0xffu;
-  const uint64_t want = ((chunk_bytes / 16 + u - 1) / u + 63) / 64 * 64;
-  if (u > 0 && want < threads) {
-    const uint32_t t2 = static_cast<uint32_t>(want < 64 ? 64 : want);
-    const uint64_t g2 = static_cast<uint64_t>(qgrid) * threads / t2;
-    qgrid = static_cast<uint32_t>(g2 < (1u << 16) ? g2 : (1u << 16));
-    if (max_grid && qgrid > max_grid) qgrid = max_grid;
-    threads = t2;
-  }
-  return launch_copy_chunks_queue(descs, static_cast<uint32_t>(n), chunk_bytes, threads, unroll,
-                                  qgrid, tiles, marks, queue, stream);
+                              s.threads, s.unroll, max_grid, stream);
+  s = queue_shape(s, chunk_bytes, is_save, table, marks != nullptr, max_grid);
+  return launch_copy_chunks_queue(descs, static_cast<uint32_t>(n), chunk_bytes, s.threads,
+                                  s.unroll, s.grid, table, marks, queue, stream);
 }
 
 // Reads back finished scatter trials; once every candidate has been timed
@@ -727,12 +701,10 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
     if (trial) PF_HIP(hipEventRecord(trial->start, stream));
   }
   unroll &= ~PF_KERNEL_AUTO;
-  QueueTiles tiles = QueueTiles::kQueue;
-  if (x->desc_base == x->h_small && n <= kQueueTableMax)
-    tiles = dir == PF_ROUTE_SAVE_HOST && !marks ? QueueTiles::kFixedTable : QueueTiles::kQueueTable;
-  const hipError_t e = issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16, host_side,
-                                  threads, unroll, qgrid, x->max_grid,
-                                  tiles, marks, queue);
+  const bool table = x->desc_base == x->h_small && n <= kQueueTableMax;
+  const hipError_t e =
+      issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16, is_save, host_side,
+                 {threads, unroll, qgrid}, x->max_grid, table, marks, queue);
   if (e != hipSuccess) return hip_fail(e, "gather/scatter kernel launch");
   if (trial) {
     PF_HIP(hipEventRecord(trial->stop, stream));
@@ -1735,9 +1707,10 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
   if (int rc = ensure_counters(x, layer_base + plans.size())) return rc;
   ChunkDesc* hd = desc_off ? nullptr : small_desc(x, total + aux_desc);
   // Host-side launches are queued, and take the whole table into LDS.
-  if (hd && total > kQueueTableMax)
+  if (hd && total > 0)
     for (const LayerPlan& p : plans)
-      if (!p.ordered && host_side_pinned(p)) hd = nullptr;
+      if (!p.ordered && !table_in_place(total, p.chunk_bytes, is_save) && host_side_pinned(p))
+        hd = nullptr;
   if (desc_off) {
     if (desc_off + total + aux_desc > x->h_cap || desc_off + total + aux_desc > x->d_cap)
       return fail(PF_ERR_INVALID_ARGUMENT, "descriptor room not reserved");
@@ -2259,10 +2232,11 @@ int pf_load_layers_noalloc(pf_stream stream, const pf_layer_xfer* layers, uint32
       const bool host = host_side_pinned(p);
       if (int rc = check_launch_size(n, p.chunk_bytes)) return rc;
       const hipError_t e = issue_copy(
-          s, d_desc + first, n, p.chunk_bytes, al, host,
-          host ? PF_LOAD_HOST_DEFAULT_THREADS : PF_LOAD_DEFAULT_THREADS,
-          host ? PF_LOAD_HOST_DEFAULT_UNROLL : (PF_LOAD_DEFAULT_UNROLL & ~PF_KERNEL_AUTO),
-          host ? PF_LOAD_HOST_DEFAULT_GRID : 0, 0, QueueTiles::kQueue, nullptr, queue);
+          s, d_desc + first, n, p.chunk_bytes, al, false, host,
+          {host ? PF_LOAD_HOST_DEFAULT_THREADS : PF_LOAD_DEFAULT_THREADS,
+           host ? PF_LOAD_HOST_DEFAULT_UNROLL : (PF_LOAD_DEFAULT_UNROLL & ~PF_KERNEL_AUTO),
+           host ? PF_LOAD_HOST_DEFAULT_GRID : 0},
+          0, false, nullptr, queue);
       if (e != hipSuccess) return hip_fail(e, "gather/scatter kernel launch");
       first += n;
       li = lj;

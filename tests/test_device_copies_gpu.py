@@ -2,7 +2,7 @@
 
 A kernel-mode save into, or load out of, a buffer in device memory moves each
 chunk as units of one wave; one that crosses the host link takes tiles from a
-queue, or by a fixed map.  The sizes here sit at the edges of a unit or a tile
+queue.  The sizes here sit at the edges of a unit or a tile
 (one wave's words, one more, one less), of a workgroup's share, of the
 descriptor table that small calls read in place, and of a launch.  The expected
 bytes are a numpy indexing of the same layout.

@@ -156,3 +156,15 @@ def test_staged_slicing_rules():
                        stderr=subprocess.STDOUT, text=True)
     assert r.returncode == 0, r.stdout[-6000:]
     assert r.stdout.strip().endswith("ok")
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is not installed")
+def test_launch_shape_rules():
+    """tests/native/launch_rules_test.cpp under AddressSanitizer+UBSan: the
+    shapes of queued launches by size, route setting and cap."""
+    exe = build("asan", "launch_rules_test")
+    env = dict(os.environ, **VARIANTS["asan"][1])
+    r = subprocess.run([exe], env=env, timeout=120, stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout[-6000:]
+    assert r.stdout.strip().endswith("ok")
