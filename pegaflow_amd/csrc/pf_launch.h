@@ -25,22 +25,27 @@ inline bool table_in_place(size_t n, uint64_t chunk_bytes, bool is_save) {
   return n <= kQueueTableMax && !(is_save && n > 512 && chunk_bytes < 4096);
 }
 
-// Workgroups of a small load, and of a marked one, whose descriptors are read
-// in place.
-constexpr uint32_t kInPlaceGrid = 16, kInPlaceMarkGrid = 32;
+// Workgroups of a load of n chunks in place on a route at its default grid.  Each
+// reads the whole table first, and a load of few bytes has no work for many:
+// with 16 and 64 workgroups, 2 MiB (64 chunks of 32 KiB) load in 61.7 and 65.3 us,
+// marked 67.4 and 70.1, 10 MiB in 208.3 and 211.3, 32 MiB in 611 and 614.  Beside
+// a save the many get more of the link, from about 8 MiB on: with 16 and 64, 2 MiB
+// take 2.5 and 2.7 ms, 10 MiB 4.3 and 2.1, 32 MiB 5.7 and 1.8, 128 MiB 12.2 and
+// 4.7.  So one a 128 KiB, at least 16.
+inline uint32_t small_load_grid(uint32_t grid, uint64_t n, uint64_t chunk_bytes) {
+  const uint64_t want = n * chunk_bytes / (128u << 10);
+  return static_cast<uint32_t>(std::min<uint64_t>(grid, std::max<uint64_t>(16, want)));
+}
 
-// The queued launch of a route set to s for chunks of chunk_bytes.  `table`: its
-// workgroups take the descriptors from host memory into LDS.  max_grid caps the
-// workgroups (0: no cap).
+// The queued launch of a route set to s for chunks of chunk_bytes.  max_grid caps
+// the workgroups (0: no cap).
 //
-// A save runs as its route says, however few its chunks.  A shape of their own
+// The route's setting holds, however few the chunks of a save.  A shape of their own
 // for small ones (8 workgroups, tiles by a fixed map, streaming stores) was as
 // fast alone (64, 320 and 1,024 chunks of 32 KiB in 62, 217-240 and 624 us, so
 // 64, 227 and 646) but ran at the pace of the XCD that a restore beside it left
 // the least of the link: 1.4, 4.4 and 12.1 ms beside one, so 0.35, 0.98 and 2.0.
-inline QueueShape queue_shape(QueueShape s, uint64_t chunk_bytes, bool is_save, bool table,
-                              bool marked, uint32_t max_grid) {
-  if (table && !is_save) s.grid = std::min(s.grid, marked ? kInPlaceMarkGrid : kInPlaceGrid);
+inline QueueShape queue_shape(QueueShape s, uint64_t chunk_bytes, uint32_t max_grid) {
   if (max_grid && s.grid > max_grid) s.grid = max_grid;
   // Chunks smaller than a tile (e.g. 4 KiB segments of one tensor-parallel
   // rank) get workgroups sized to the chunk, and proportionally more of

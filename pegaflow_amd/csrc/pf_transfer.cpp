@@ -595,13 +595,13 @@ ChunkDesc* small_desc(pf_xfer* x, size_t n) {
 // memory.  Otherwise a fixed map hands out units (at most max_grid workgroups,
 // 0 = no cap).
 hipError_t issue_copy(hipStream_t stream, const ChunkDesc* descs, size_t n, uint64_t chunk_bytes,
-                      bool al16, bool is_save, bool host_side, QueueShape s, uint32_t max_grid,
-                      bool table, const LayerMarks* marks, uint32_t* queue) {
+                      bool al16, bool host_side, QueueShape s, uint32_t max_grid, bool table,
+                      const LayerMarks* marks, uint32_t* queue) {
   (void)hipGetLastError();
   if (!(al16 && s.grid > 0))
     return launch_copy_chunks(descs, static_cast<uint32_t>(n), chunk_bytes, al16, host_side,
                               s.threads, s.unroll, max_grid, stream);
-  s = queue_shape(s, chunk_bytes, is_save, table, marks != nullptr, max_grid);
+  s = queue_shape(s, chunk_bytes, max_grid);
   return launch_copy_chunks_queue(descs, static_cast<uint32_t>(n), chunk_bytes, s.threads,
                                   s.unroll, s.grid, table, marks, queue, stream);
 }
@@ -685,7 +685,6 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
   // (its layers must land in order).  See copy_chunks_queue_kernel.
   uint32_t qgrid = x->grid[dir];
   if (marks && qgrid == 0) qgrid = PF_LOAD_HOST_DEFAULT_GRID;
-  if (x->max_grid && qgrid > x->max_grid) qgrid = x->max_grid;
   // Each lane's launches run in its stream's order; the two lanes overlap.
   uint32_t* queue = x->d_queue[stream == x->dma ? 1 : 0];
   if (al16 && qgrid > 0 && !queue)
@@ -702,8 +701,10 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
   }
   unroll &= ~PF_KERNEL_AUTO;
   const bool table = x->desc_base == x->h_small && n <= kQueueTableMax;
+  if (table && dir == PF_ROUTE_LOAD_HOST && qgrid == PF_LOAD_HOST_DEFAULT_GRID)
+    qgrid = small_load_grid(qgrid, n, chunk_bytes);
   const hipError_t e =
-      issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16, is_save, host_side,
+      issue_copy(stream, x->desc_base + first, n, chunk_bytes, al16, host_side,
                  {threads, unroll, qgrid}, x->max_grid, table, marks, queue);
   if (e != hipSuccess) return hip_fail(e, "gather/scatter kernel launch");
   if (trial) {
@@ -2232,7 +2233,7 @@ int pf_load_layers_noalloc(pf_stream stream, const pf_layer_xfer* layers, uint32
       const bool host = host_side_pinned(p);
       if (int rc = check_launch_size(n, p.chunk_bytes)) return rc;
       const hipError_t e = issue_copy(
-          s, d_desc + first, n, p.chunk_bytes, al, false, host,
+          s, d_desc + first, n, p.chunk_bytes, al, host,
           {host ? PF_LOAD_HOST_DEFAULT_THREADS : PF_LOAD_DEFAULT_THREADS,
            host ? PF_LOAD_HOST_DEFAULT_UNROLL : (PF_LOAD_DEFAULT_UNROLL & ~PF_KERNEL_AUTO),
            host ? PF_LOAD_HOST_DEFAULT_GRID : 0},

@@ -1,7 +1,7 @@
 // launch_rules_test.cpp — the launch shapes' rules (pf_launch.h) on the host
 // (no GPU), built by tests/test_native.py from the library's own sources:
-//   * a queued save keeps its route's workgroups, loads in flight and flags,
-//     with its descriptors in place or not;
+//   * a queued launch keeps its route's workgroups, loads in flight and flags;
+//   * a small load at the default grid: workgroups by its bytes;
 //   * the calls over the host link whose descriptors are read in place;
 //   * chunks smaller than a tile: workgroups of the chunk's size, as many
 //     lanes in all, within the caps.
@@ -36,24 +36,25 @@ void same(const QueueShape& got, const QueueShape& want, const std::string& what
 int main() {
   const QueueShape save{PF_SAVE_HOST_DEFAULT_THREADS, PF_SAVE_HOST_DEFAULT_UNROLL,
                         PF_SAVE_HOST_DEFAULT_GRID};
-  for (bool table : {false, true}) {
-    const std::string where = table ? " in place" : " uploaded";
-    same(queue_shape(save, 32768, true, table, false, 0), save, "default save" + where);
-    for (uint32_t grid : {1u, 3u, 32u, 64u, 5000u}) {
-      const QueueShape s{256, 4u | PF_KERNEL_NT_LOADS, grid};
-      same(queue_shape(s, 131072, true, table, false, 0), s,
-           "save of " + std::to_string(grid) + " workgroups" + where);
-      same(queue_shape(s, 131072, true, table, false, 7), {256, s.unroll, grid < 7 ? grid : 7},
-           "capped save of " + std::to_string(grid) + " workgroups" + where);
-    }
-    // A 4 KiB chunk is 128 lanes of two words, a 16-byte one a wave.
-    same(queue_shape(save, 4096, true, table, false, 0), {128, save.unroll, 128},
-         "save of 4 KiB chunks" + where);
-    same(queue_shape(save, 4096, true, table, false, 100), {128, save.unroll, 100},
-         "capped save of 4 KiB chunks" + where);
-    same(queue_shape({512, 2, 1u << 20}, 16, true, table, false, 0), {64, 2, 1u << 16},
-         "save of 16-byte chunks" + where);
+  same(queue_shape(save, 32768, 0), save, "default save");
+  for (uint32_t grid : {1u, 3u, 32u, 64u, 5000u}) {
+    const QueueShape s{256, 4u | PF_KERNEL_NT_LOADS, grid};
+    const std::string what = std::to_string(grid) + " workgroups";
+    same(queue_shape(s, 131072, 0), s, what);
+    same(queue_shape(s, 131072, 7), {256, s.unroll, grid < 7 ? grid : 7}, what + ", capped");
   }
+  // A 4 KiB chunk is 128 lanes of two words, a 16-byte one a wave.
+  same(queue_shape(save, 4096, 0), {128, save.unroll, 128}, "4 KiB chunks");
+  same(queue_shape(save, 4096, 100), {128, save.unroll, 100}, "4 KiB chunks, capped");
+  same(queue_shape({512, 2, 1u << 20}, 16, 0), {64, 2, 1u << 16}, "16-byte chunks");
+  // A small load's workgroups: 16 up to 2 MiB, the route's 64 from 8 MiB on.
+  const uint64_t loads[][3] = {{1, 16, 16}, {64, 32768, 16}, {64, 36864, 18}, {128, 32768, 32},
+                               {255, 32768, 63}, {256, 32768, 64}, {1024, 131072, 64},
+                               {1, 1ull << 34, 64}};
+  for (const auto& t : loads)
+    expect(small_load_grid(PF_LOAD_HOST_DEFAULT_GRID, t[0], t[1]) == t[2],
+           "load of " + std::to_string(t[0]) + " chunks of " + std::to_string(t[1]));
+  expect(small_load_grid(3, 64, 32768) == 3, "no more workgroups than the route's");
   for (bool is_save : {false, true}) {
     const std::string what = is_save ? "save in place" : "load in place";
     expect(table_in_place(1, 16, is_save) && table_in_place(512, 16, is_save), what);

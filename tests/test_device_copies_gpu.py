@@ -169,6 +169,41 @@ def test_small_host_copies(gpu, bpb, segs, counts):
     ctx.close()
 
 
+# Chunks whose descriptors are read in place, and more than are.
+@pytest.mark.parametrize("n", [8, 1100])
+def test_more_workgroups_than_tiles(gpu, n):
+    """A queue that most workgroups find empty, call after call: save, load and marked
+    load, and between device buffers on routes that are set to run queued."""
+    (layer,) = make_layers(np.random.default_rng(n), 1040, 1, (n,), n + 3)
+    words = PinnedBuffer(8)
+    words.array[:] = 0
+    ctx = TransferContext(0)
+    for route in (_lib.ROUTE_SAVE_HOST, _lib.ROUTE_LOAD_HOST, _lib.ROUTE_SAVE_DEVICE,
+                  _lib.ROUTE_LOAD_DEVICE):
+        ctx.set_route_grid(route, 5000)
+    host, device = PinnedBuffer(layer.nbytes), DeviceBuffer(layer.nbytes)
+    for value in (1, 2, 3):
+        for pool in (host, device):
+            xfer = layer.transfer(pool.ptr)
+            ctx.save_layers([xfer], _lib.MODE_KERNEL)
+            got = pool.array if pool is host else pool.download()
+            assert np.array_equal(got, layer.packed())
+            packed = np.random.default_rng(value).integers(0, 256, layer.nbytes, np.uint8)
+            if pool is host:
+                pool.array[:] = packed
+            else:
+                pool.upload(packed)
+            if pool is host and value == 2:
+                ctx.load_layers_marked([xfer], [(words.ptr, value, True)], _lib.MODE_KERNEL)
+            else:
+                ctx.load_layers([xfer], _lib.MODE_KERNEL)
+            ctx.synchronize()
+            layer.restore(packed)
+            assert np.array_equal(layer.dev.download(), layer.host)
+    assert words.array.view(np.uint64).tolist() == [2]
+    ctx.close()
+
+
 # Chunks shorter than a word, around one, around a unit, and of several units, at
 # every kind of offset from a word's boundary.
 UNALIGNED = [(bpb, off) for bpb in (1, 7, 15, 16, 17, 33, 200, 1009, 1023, 1025, 1041, 2060, 12301)
