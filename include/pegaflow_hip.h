@@ -369,7 +369,8 @@ int pf_xfer_route_shape(pf_xfer* xfer, uint32_t route, uint32_t* threads,
  * a marked load's layers, finishing in order, and few requests in flight
  * keep the link at its peak).  Marked launches out of pinned host memory
  * always run queued (at PF_LOAD_HOST_DEFAULT_GRID when their route says 0);
- * marked copies between device buffers have a workgroup per 8 or 32 KiB.  A
+ * marked copies between device buffers have a workgroup per up to 8 or 32 KiB
+ * of a layer.  A
  * load of up to 1,024 chunks and 8 MiB on a route at PF_LOAD_HOST_DEFAULT_GRID
  * runs with one workgroup a 128 KiB, at least 16; any other setting holds as it
  * is.  pf_xfer_set_max_grid caps both kinds.  Every route may run queued: the
@@ -506,15 +507,16 @@ int pf_load_layers_noalloc(pf_stream stream, const pf_layer_xfer* layers,
  * gpu_worker.rs:286-291).  Unlike layer_events, marks do not split a load
  * from pinned host memory into one launch per layer: in PF_MODE_KERNEL one
  * launch covers every such layer (two for a large call, whose first eighth
- * of layers is launched before the rest is planned) and its last workgroup
- * on layer l writes the marks of layer l.  Layers loaded from device memory (an
- * HBM-bound copy) get one launch each, followed by their marks; DMA copies
- * are marked after each layer's copies.  In PF_MODE_STAGED (and AUTO when it
- * stages) each slice's scatter marks the layers it completes, counting a
+ * of layers, first quarter of a copy out of device memory, is launched before
+ * the rest is planned) and its last workgroup on layer l writes the marks of
+ * layer l.  Layers whose chunks are not all 16-byte aligned share a launch too,
+ * marked as they land out of device memory, after the launch out of pinned host
+ * memory; DMA copies are marked after each layer's copies.  In PF_MODE_STAGED
+ * (and AUTO when it stages) each slice's scatter marks the layers it completes, counting a
  * layer's tiles over the slices that hold it, so a layer lands after one
  * kernel; layers in slices that cannot carry them (more than 8 layers,
  * unaligned chunks) are marked by a separate kernel after their last
- * slice. 
+ * slice.
  *
  * A signal target is an array of one 8-byte word per layer of the call:
  * words + 8*l is set to `value` once layer l's bytes are in place.  The

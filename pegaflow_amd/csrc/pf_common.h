@@ -73,20 +73,25 @@ struct LayerMarks {
 };
 
 // A marked copy between device buffers works in units of up to 64 *
-// kMarkedUnroll 16-byte words of one chunk, one wave each; a workgroup of
-// kMarkedThreads takes up to 4 * loops consecutive units of one layer.
+// kMarkedUnroll 16-byte words of one chunk (64 words of an unaligned one), one
+// wave each; a workgroup of kMarkedThreads takes up to wg_units consecutive
+// units of one layer.
 constexpr uint32_t kMarkedThreads = 256;
 constexpr uint32_t kMarkedUnroll = 2;
 struct MarkedShape {
   uint32_t units_per_chunk;
   uint32_t wg_units;  // units of one workgroup
 };
-inline MarkedShape marked_shape(uint64_t chunk_bytes, uint64_t launch_chunks) {
-  const uint64_t unit = 64ull * kMarkedUnroll * 16;
-  // 32 KiB a workgroup, and 8 KiB in launches too small to fill the chip
+inline MarkedShape marked_shape(uint64_t chunk_bytes, uint64_t launch_chunks, bool aligned) {
+  const uint64_t unit = 64ull * 16 * (aligned ? kMarkedUnroll : 1);
+  // Up to 32 KiB a workgroup, and 8 KiB in launches too small to fill the chip
   // with those (see copy_chunks_marked_kernel).
-  const uint32_t loops = launch_chunks * chunk_bytes >= (32ull << 20) ? 4 : 1;
-  return {static_cast<uint32_t>((chunk_bytes + unit - 1) / unit), kMarkedThreads / 64 * loops};
+  const uint64_t share = launch_chunks * chunk_bytes >= (32ull << 20) ? 32768 : 8192;
+  // An unaligned chunk's words lie between its first and last few bytes, and a
+  // chunk of those only still has a unit.
+  const uint64_t units = aligned ? (chunk_bytes + unit - 1) / unit
+                                 : (chunk_bytes < 16 ? 1 : (chunk_bytes / 16 + 63) / 64);
+  return {static_cast<uint32_t>(units), static_cast<uint32_t>(share / unit)};
 }
 // Workgroups of a layer's `chunks` chunks in one launch.
 inline uint64_t marked_workgroups(const MarkedShape& s, uint64_t chunks) {
@@ -145,16 +150,17 @@ hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint64_t chunk_bytes, uint32_t threads, uint32_t unroll,
                                     uint32_t grid, bool table, const LayerMarks* marks,
                                     uint32_t* queue, hipStream_t stream);
-// A marked copy between device buffers (16-byte aligned chunks): each finished
-// layer of the marks is marked.  At most max_grid workgroups (0: no cap).  The
-// table's n_wg workgroups and its entries are those of marked_shape(chunk_bytes,
-// n_chunks) over its layers.
+// A marked copy between device buffers: each finished layer of the marks is
+// marked.  At most max_grid workgroups (0: no cap).  The table's n_wg workgroups
+// and its entries are those of marked_shape(chunk_bytes, n_chunks, aligned16) over
+// its layers; marks by value need 16-byte aligned chunks.
 hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks,
                                      uint64_t chunk_bytes, uint32_t max_grid, SliceMarks marks,
                                      hipStream_t stream);
 hipError_t launch_copy_chunks_mark_table(const ChunkDesc* d_descs, uint32_t n_chunks,
-                                         uint64_t chunk_bytes, uint32_t n_wg, uint32_t max_grid,
-                                         const MarkTable& marks, hipStream_t stream);
+                                         uint64_t chunk_bytes, bool aligned16, uint32_t n_wg,
+                                         uint32_t max_grid, const MarkTable& marks,
+                                         hipStream_t stream);
 hipError_t launch_mark_layers(const LayerList& list, const SignalTargets& t,
                               hipStream_t stream);
 hipError_t launch_wait_word(uint64_t word, uint64_t value, uint64_t max_ticks,

@@ -193,6 +193,38 @@ __device__ __forceinline__ void store16_through(uint64_t base, uint32_t bytes, u
   __builtin_amdgcn_raw_buffer_store_b128(v, r, static_cast<int>(lane * 16), 0, kSc1);
 }
 
+// Unit u of a chunk whose addresses or size are not 16-byte aligned.  A chunk's
+// stores are 16-byte words at aligned addresses, its loads the 16 bytes that go
+// there, at whatever address they have; up to 15 bytes in front of the first
+// word go with the chunk's first unit and those behind the last word with its
+// last (THROUGH: written through the L2, as the words are).
+template <bool THROUGH>
+__device__ __forceinline__ void copy_unaligned_unit(const ChunkDesc& d, uint32_t u,
+                                                    uint32_t units_per_chunk, uint64_t chunk_bytes,
+                                                    uint32_t lane) {
+  const uint64_t to_word = (16u - (d.dst & 15u)) & 15u;
+  const uint64_t head = to_word < chunk_bytes ? to_word : chunk_bytes;
+  const uint64_t words = (chunk_bytes - head) >> 4;  // <= 64 * units_per_chunk
+  const uint32_t tail = static_cast<uint32_t>(chunk_bytes - head) & 15u;
+  const uint64_t src = d.src + head, dst = d.dst + head;
+  const uint64_t e0 = static_cast<uint64_t>(u) * 64u;
+  auto byte = [&](uint64_t to, uint64_t from) {
+    const uint8_t v = *reinterpret_cast<const g_u8*>(from);
+    if constexpr (THROUGH)
+      __hip_atomic_store(reinterpret_cast<g_u8*>(to), v, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    else
+      *reinterpret_cast<g_u8*>(to) = v;
+  };
+  if (e0 + lane < words)
+    store16_through(dst + e0 * 16u, 1024u, lane,
+                    __builtin_nontemporal_load(reinterpret_cast<const g_u32x4_any*>(src) + e0 +
+                                               lane));
+  if (u == 0 && lane < head) byte(d.dst + lane, d.src + lane);
+  if (u == units_per_chunk - 1 && lane < tail)
+    byte(dst + words * 16u + lane, src + words * 16u + lane);
+}
+
 // A marked copy between device buffers: the device-sourced marked load (one
 // launch over its layers, table in device memory) and the staged load's
 // scatter of a slice whose layers it reports itself (table in the arguments).
@@ -213,10 +245,16 @@ __device__ __forceinline__ void store16_through(uint64_t base, uint32_t bytes, u
 // each before, took 450 us, here 94 in one launch.  A launch of a single 40 MiB
 // layer (a staged slice, under the next slice's copy) is bound by its 1,280 adds
 // to one counter: 28.7 us, where 128 workgroups with fences took 24.0.
-template <int UNROLL, class Marks>
+//
+// Chunks that are not aligned (ALIGNED false) go by units of 64 words, their odd
+// bytes written through as well: 61 layers of 4.7 MB in 36,865-byte chunks land
+// one by one in 163 us a call (one unmarked launch, every layer marked behind it,
+// 155; a byte-wise launch a layer 2,123).
+template <int UNROLL, bool ALIGNED, class Marks>
 __global__ void __launch_bounds__(kMarkedThreads)
 copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape,
-                          uint32_t chunk16, uint32_t n_wg, Marks marks) {
+                          uint64_t chunk_bytes, uint32_t n_wg, Marks marks) {
+  const uint32_t chunk16 = static_cast<uint32_t>(chunk_bytes / 16);
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr uint32_t kWaves = kMarkedThreads / 64;
@@ -229,20 +267,25 @@ copy_chunks_marked_kernel(const ChunkDesc* __restrict__ descs, MarkedShape shape
     for (uint32_t i = wave; i < mine; i += kWaves) {
       const uint32_t unit = first + i;
       const uint32_t c = unit / shape.units_per_chunk;
-      const uint32_t e0 = (unit - c * shape.units_per_chunk) * (64u * UNROLL);
+      const uint32_t in_chunk = unit - c * shape.units_per_chunk;
       const ChunkDesc d = descs[g.chunk_start + c];
-      const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src) + e0;
-      const uint32_t words = chunk16 - e0;  // of this unit and what follows it
-      u32x4 v[UNROLL];
+      if constexpr (!ALIGNED) {
+        copy_unaligned_unit<true>(d, in_chunk, shape.units_per_chunk, chunk_bytes, lane);
+      } else {
+        const uint32_t e0 = in_chunk * (64u * UNROLL);
+        const g_u32x4* __restrict__ src = reinterpret_cast<const g_u32x4*>(d.src) + e0;
+        const uint32_t words = chunk16 - e0;  // of this unit and what follows it
+        u32x4 v[UNROLL];
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u)
-        if (u * 64u + lane < words) v[u] = load16<true>(src + u * 64u + lane);
+        for (int u = 0; u < UNROLL; ++u)
+          if (u * 64u + lane < words) v[u] = load16<true>(src + u * 64u + lane);
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if (u * 64u >= words) break;
-        const uint32_t n = words - u * 64u;
-        store16_through(d.dst + (static_cast<uint64_t>(e0) + u * 64u) * 16u,
-                        (n < 64u ? n : 64u) * 16u, lane, v[u]);
+        for (int u = 0; u < UNROLL; ++u) {
+          if (u * 64u >= words) break;
+          const uint32_t n = words - u * 64u;
+          store16_through(d.dst + (static_cast<uint64_t>(e0) + u * 64u) * 16u,
+                          (n < 64u ? n : 64u) * 16u, lane, v[u]);
+        }
       }
     }
     if (g.units == 0) continue;  // marked by another kernel (uniform: no barrier is missed)
@@ -474,13 +517,9 @@ copy_chunks_b1_kernel(const ChunkDesc* __restrict__ descs, uint32_t n_chunks,
   }
 }
 
-// The same between device buffers, by units as in the fixed map.  A chunk's
-// stores are 16-byte words at aligned addresses, its loads the 16 bytes that go
-// there, at whatever address they have; up to 15 bytes in front of the first
-// word go with the chunk's first unit and those behind the last word with its
-// last.  Bound by HBM: 59 MB in 12,300-byte chunks take 27 us, byte by byte 61;
-// 200-byte chunks 66 and 115.  (Aligned loads shifted between the lanes were no
-// faster.)
+// The same between device buffers, by units as in the fixed map.  Bound by HBM:
+// 59 MB in 12,300-byte chunks take 27 us, byte by byte 61; 200-byte chunks 66 and
+// 115.  (Aligned loads shifted between the lanes were no faster.)
 __global__ void __launch_bounds__(kFixedThreads)
 copy_chunks_unaligned_kernel(const ChunkDesc* __restrict__ descs, uint32_t units_per_chunk,
                              uint32_t n_units, uint64_t chunk_bytes) {
@@ -492,23 +531,8 @@ copy_chunks_unaligned_kernel(const ChunkDesc* __restrict__ descs, uint32_t units
         __builtin_amdgcn_readfirstlane(b * waves + (threadIdx.x >> 6));
     if (unit >= n_units) continue;
     const uint32_t c = unit / units_per_chunk;
-    const uint32_t u = unit - c * units_per_chunk;
-    const ChunkDesc d = descs[c];
-    const uint64_t to_word = (16u - (d.dst & 15u)) & 15u;
-    const uint64_t head = to_word < chunk_bytes ? to_word : chunk_bytes;
-    const uint64_t words = (chunk_bytes - head) >> 4;  // <= 64 * units_per_chunk
-    const uint32_t tail = static_cast<uint32_t>(chunk_bytes - head) & 15u;
-    const uint64_t src = d.src + head, dst = d.dst + head;
-    const uint64_t e0 = static_cast<uint64_t>(u) * 64u;
-    if (e0 + lane < words)
-      store16_through(dst + e0 * 16u, 1024u, lane,
-                      __builtin_nontemporal_load(
-                          reinterpret_cast<const g_u32x4_any*>(src) + e0 + lane));
-    if (u == 0 && lane < head)
-      reinterpret_cast<g_u8*>(d.dst)[lane] = reinterpret_cast<const g_u8*>(d.src)[lane];
-    if (u == units_per_chunk - 1 && lane < tail)
-      reinterpret_cast<g_u8*>(dst + words * 16u)[lane] =
-          reinterpret_cast<const g_u8*>(src + words * 16u)[lane];
+    copy_unaligned_unit<false>(descs[c], unit - c * units_per_chunk, units_per_chunk, chunk_bytes,
+                               lane);
   }
 }
 
@@ -691,21 +715,21 @@ hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
 // Every unit of a marked launch lies in its chunk: chunk16 < 2^31, and the
 // units of a launch are counted in 32 bits.
 static bool marked_fits(const MarkedShape& s, uint32_t n_chunks, uint64_t chunk_bytes,
-                        uint64_t n_wg) {
-  return chunk_bytes % 16 == 0 && chunk_bytes / 16 < (1ull << 31) &&
+                        bool aligned16, uint64_t n_wg) {
+  return !(aligned16 && chunk_bytes % 16) && chunk_bytes / 16 < (1ull << 31) &&
          static_cast<uint64_t>(n_chunks) * s.units_per_chunk + s.wg_units <= 0xffffffffull &&
          n_wg > 0 && n_wg + kMaxGrid <= 0xffffffffull;
 }
 
-template <class Marks>
+template <bool ALIGNED, class Marks>
 static hipError_t launch_marked(const ChunkDesc* d_descs, uint64_t chunk_bytes,
                                 const MarkedShape& s, uint32_t n_wg, uint32_t max_grid,
                                 const Marks& marks, hipStream_t stream) {
   uint32_t cap = max_grid ? max_grid : kMaxGrid;
   if (cap > kMaxGrid) cap = kMaxGrid;
-  hipLaunchKernelGGL((copy_chunks_marked_kernel<kMarkedUnroll, Marks>),
+  hipLaunchKernelGGL((copy_chunks_marked_kernel<kMarkedUnroll, ALIGNED, Marks>),
                      dim3(n_wg < cap ? n_wg : cap), dim3(kMarkedThreads), 0, stream, d_descs, s,
-                     static_cast<uint32_t>(chunk_bytes / 16), n_wg, marks);
+                     chunk_bytes, n_wg, marks);
   return hipGetLastError();
 }
 
@@ -717,7 +741,7 @@ hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks
       marks.targets.count == 0 || marks.targets.count > kMaxSignalTargets ||
       marks.chunk_start[0] != 0 || marks.chunk_start[marks.n] != n_chunks)
     return hipErrorInvalidValue;
-  const MarkedShape s = marked_shape(chunk_bytes, n_chunks);
+  const MarkedShape s = marked_shape(chunk_bytes, n_chunks, true);
   // Groups in chunk order, each counting at least its own units.
   uint64_t wg = 0;
   for (uint32_t g = 0; g < marks.n; ++g) {
@@ -728,22 +752,24 @@ hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks
     marks.wg_start[g] = static_cast<uint32_t>(wg);
     wg += marked_workgroups(s, chunks);
   }
-  if (!marked_fits(s, n_chunks, chunk_bytes, wg)) return hipErrorInvalidValue;
+  if (!marked_fits(s, n_chunks, chunk_bytes, true, wg)) return hipErrorInvalidValue;
   marks.wg_start[marks.n] = static_cast<uint32_t>(wg);
-  return launch_marked(d_descs, chunk_bytes, s, static_cast<uint32_t>(wg), max_grid, marks,
-                       stream);
+  return launch_marked<true>(d_descs, chunk_bytes, s, static_cast<uint32_t>(wg), max_grid, marks,
+                             stream);
 }
 
 hipError_t launch_copy_chunks_mark_table(const ChunkDesc* d_descs, uint32_t n_chunks,
-                                         uint64_t chunk_bytes, uint32_t n_wg, uint32_t max_grid,
-                                         const MarkTable& marks, hipStream_t stream) {
+                                         uint64_t chunk_bytes, bool aligned16, uint32_t n_wg,
+                                         uint32_t max_grid, const MarkTable& marks,
+                                         hipStream_t stream) {
   if (n_chunks == 0 || chunk_bytes == 0) return hipSuccess;
   if (marks.n == 0 || !marks.wg_start || !marks.chunk_start || !marks.layer || !marks.counters ||
       marks.targets.count == 0 || marks.targets.count > kMaxSignalTargets)
     return hipErrorInvalidValue;
-  const MarkedShape s = marked_shape(chunk_bytes, n_chunks);
-  if (!marked_fits(s, n_chunks, chunk_bytes, n_wg)) return hipErrorInvalidValue;
-  return launch_marked(d_descs, chunk_bytes, s, n_wg, max_grid, marks, stream);
+  const MarkedShape s = marked_shape(chunk_bytes, n_chunks, aligned16);
+  if (!marked_fits(s, n_chunks, chunk_bytes, aligned16, n_wg)) return hipErrorInvalidValue;
+  return aligned16 ? launch_marked<true>(d_descs, chunk_bytes, s, n_wg, max_grid, marks, stream)
+                   : launch_marked<false>(d_descs, chunk_bytes, s, n_wg, max_grid, marks, stream);
 }
 
 hipError_t launch_mark_layers(const LayerList& list, const SignalTargets& t,

@@ -717,8 +717,7 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
   return PF_OK;
 }
 
-// A marked copy between device buffers (16-byte aligned chunks) on the
-// context's stream: launch_it(descriptors, stream) issues it.
+// A marked copy between device buffers on the context's stream: launch_it(descriptors, stream) issues it.
 template <class F>
 int launch_marked_copy(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, F launch_it) {
   if (n == 0) return PF_OK;
@@ -1207,7 +1206,7 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
         m.chunk_start[m.n + 1] = m.chunk_start[m.n] + static_cast<uint32_t>(pc.end - pc.begin);
         if (self_marked[pc.layer] == 1) {
           m.units[m.n] = static_cast<uint32_t>(
-              p.chunks.size() * marked_shape(p.chunk_bytes, st.n_chunks).units_per_chunk);
+              p.chunks.size() * marked_shape(p.chunk_bytes, st.n_chunks, true).units_per_chunk);
           counts = true;
         }
         ++m.n;
@@ -1659,9 +1658,9 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
       continue;
     }
     const bool al = chunks_aligned(p);
-    // A marked launch is queued when its sources are pinned host memory, and
-    // a marked device copy when they are device memory: one launch holds
-    // layers of one kind.
+    // A marked launch is queued when its sources are pinned host memory (and
+    // aligned), and a marked device copy when they are device memory: one
+    // launch holds layers of one kind.
     const bool host_src = !p.chunks.empty() && host_sourced(p, is_save);
     size_t lj = li + 1;
     if (!layer_events) {
@@ -1673,11 +1672,11 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
         ++lj;
     }
     Step st{li, lj, false, al};
-    if (sig && al && !layer_events) {
+    if (sig && (al || !host_src) && !layer_events) {
       st.tab = aux.size();
       size_t chunks = 0;
       for (size_t k = li; k < lj; ++k) chunks += plans[k].chunks.size();
-      const MarkedShape shape = marked_shape(p.chunk_bytes, chunks);
+      const MarkedShape shape = marked_shape(p.chunk_bytes, chunks, al);
       std::vector<uint32_t> ids, wg_start;
       uint64_t start = 0, wgs = 0;
       for (size_t k = li; k < lj; ++k) {
@@ -1759,8 +1758,8 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
       const uint64_t cb = plans[st.li].chunk_bytes;
       if (int rc = launch_marked_copy(
               x, first[st.li], n, cb, [&](const ChunkDesc* dd, hipStream_t s) {
-                return launch_copy_chunks_mark_table(dd, static_cast<uint32_t>(n), cb, st.wgs,
-                                                     x->max_grid, t, s);
+                return launch_copy_chunks_mark_table(dd, static_cast<uint32_t>(n), cb, st.aligned,
+                                                     st.wgs, x->max_grid, t, s);
               }))
         return rc;
     } else {
@@ -1786,7 +1785,8 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     if (layer_events && layer_events[st.li])
       PF_HIP(hipEventRecord(static_cast<hipEvent_t>(layer_events[st.li]), x->stream));
     if (sig) {
-      // Layers the launch did not mark: empty ones, and all of an unaligned launch.
+      // Layers the launch did not mark: empty ones, and all of an unaligned launch
+      // over the host link.
       std::vector<uint32_t> rest;
       for (size_t k = st.li; k < st.lj; ++k)
         if (!marked || plans[k].chunks.empty())

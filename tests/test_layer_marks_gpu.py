@@ -15,6 +15,7 @@ device 0 through the C ABI:
 """
 
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -280,6 +281,107 @@ def test_device_wait_orders_consumer_per_layer(ctx):
         host_words.close()
         dev_words.close()
         flag.close()
+
+
+class MarkedCopies:
+    """8 layers of 1,000 blocks each (2 x 64 KiB, or a byte more) out of a pool into
+    tensors of 1,100: in random order, but for the last 16, whose places in the layer's
+    second segment are its end, as they are in the pool."""
+
+    def __init__(self, pool, bpb):
+        rng = np.random.Generator(np.random.PCG64(bpb))
+        nb, n, self.layers, self.tail = 1100, 1000, 8, 16 * bpb
+        self.pool, self.payload = pool(8 * 2 * n * bpb), 2 * n * bpb
+        self.bufs = [DeviceBuffer((2 * nb * bpb + 7) // 8 * 8) for _ in range(self.layers)]
+        self.end, self.ids = 2 * nb * bpb, []
+        self.transfers = []
+        for l, buf in enumerate(self.bufs):
+            buf.memset(0)
+            reg = KVCacheRegistration.create(buf.ptr, 2 * nb * bpb, nb, bpb, nb * bpb, 2)
+            ids = np.concatenate([rng.permutation(nb - 16)[:n - 16], np.arange(nb - 16, nb)])
+            k = self.pool.ptr + l * self.payload + np.arange(n, dtype=np.uint64) * np.uint64(bpb)
+            self.ids.append(ids)
+            self.transfers.append(LayerTransfer(reg, block_array(ids, k, k + np.uint64(n * bpb))))
+        self.bpb, self.nb = bpb, nb
+
+    def refill(self, seed):
+        if isinstance(self.pool, PinnedBuffer):
+            self.pool.array[:] = np.random.default_rng(seed).integers(0, 256, self.pool.nbytes,
+                                                                      np.uint8)
+            self.host = self.pool.array
+        else:
+            self.pool.fill_random(seed)
+            self.host = self.pool.download()
+
+    def check(self, layer):
+        """Every byte of a layer, the blocks that were not loaded included."""
+        want = np.zeros((2, self.nb, self.bpb), np.uint8)
+        at = layer * self.payload
+        want[:, self.ids[layer]] = self.host[at:at + self.payload].reshape(2, -1, self.bpb)
+        assert np.array_equal(self.bufs[layer].download(self.end), want.reshape(-1))
+
+    def close(self):
+        for b in (*self.bufs, self.pool):
+            b.close()
+
+
+MARKED_COPIES = {"device": (DeviceBuffer, 65536, "kernel"),
+                 "device_unaligned": (DeviceBuffer, 65537, "kernel"),
+                 "staged": (PinnedBuffer, 65536, "staged")}
+
+
+@pytest.mark.parametrize("kind", list(MARKED_COPIES))
+def test_marked_copies_land_layer_by_layer(gpu, kind):
+    """A load of 1 GB whose copies mark their layers themselves: the host sees the first
+    layer's word while the last one's is not set (0.3 ms later at the least), and a consumer
+    stream that waits on each layer's device word finds the last bytes that the copy wrote
+    of it (a layer is 131 MB: what the kernel has not yet written, or has left in some L2,
+    would be missing)."""
+    say(f"[gpu] marked copies, layer by layer: {kind}")
+    pool, bpb, mode = MARKED_COPIES[kind]
+    x = TransferContext(0, staging_bytes=512 * MiB if mode == "staged" else 0)
+    c = MarkedCopies(pool, bpb)
+    L = c.layers
+    host_words, dev_words, flag = PinnedBuffer(8 * L), DeviceBuffer(8 * L), DeviceBuffer(4 * L)
+    snaps = [DeviceBuffer(c.tail) for _ in range(L)]
+    words = host_words.array.view(np.uint64)
+    words[:] = 0
+    dev_words.memset(0)
+    flag.memset(0)
+    consumer = Stream()
+    targets = lambda v: [(host_words.ptr, v, True), (dev_words.ptr, v, False)]
+    try:
+        c.refill(1)
+        x.load_layers_marked(c.transfers, targets(1), MODES[mode])
+        seen, end = [words.tolist()], time.monotonic() + 10
+        while seen[-1] != [1] * L and time.monotonic() < end:
+            now = words.tolist()
+            if now != seen[-1]:
+                seen.append(now)
+        x.synchronize()
+        for l in range(L):
+            c.check(l)
+        assert seen[-1] == [1] * L
+        assert any(s[0] == 1 and s[-1] == 0 for s in seen), f"words came together: {seen}"
+        for value in (2, 3):
+            c.refill(value)
+            x.load_layers_marked(c.transfers, targets(value), MODES[mode])
+            for l in range(L):
+                stream_wait_word(consumer, dev_words.ptr + 8 * l, value, 10_000_000,
+                                 flag.ptr + 4 * l)
+                memcpy_async(snaps[l].ptr, c.bufs[l].ptr + c.end - c.tail, c.tail, consumer)
+            consumer.synchronize()
+            x.synchronize()
+            assert not flag.download().any(), "a device wait timed out"
+            for l in range(L):
+                at = (l + 1) * c.payload
+                assert np.array_equal(snaps[l].download(), c.host[at - c.tail:at]), f"layer {l}"
+    finally:
+        consumer.close()
+        x.close()
+        c.close()
+        for b in (host_words, dev_words, flag, *snaps):
+            b.close()
 
 
 def test_bounded_wait_times_out(gpu):
