@@ -1672,7 +1672,7 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
         ++lj;
     }
     Step st{li, lj, false, al};
-    if (sig && (al || !host_src) && !layer_events) {
+    if (sig && (al || !host_src) && p.chunk_bytes > 0 && !layer_events) {
       st.tab = aux.size();
       size_t chunks = 0;
       for (size_t k = li; k < lj; ++k) chunks += plans[k].chunks.size();
@@ -1786,7 +1786,7 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
       PF_HIP(hipEventRecord(static_cast<hipEvent_t>(layer_events[st.li]), x->stream));
     if (sig) {
       // Layers the launch did not mark: empty ones, and all of an unaligned launch
-      // over the host link.
+      // over the host link or of one with no bytes to copy.
       std::vector<uint32_t> rest;
       for (size_t k = st.li; k < st.lj; ++k)
         if (!marked || plans[k].chunks.empty())

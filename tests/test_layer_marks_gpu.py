@@ -14,6 +14,7 @@ device 0 through the C ABI:
   * the bounded wait ends on its time limit when the word is never set.
 """
 
+import dataclasses
 import sys
 import time
 
@@ -281,6 +282,26 @@ def test_device_wait_orders_consumer_per_layer(ctx):
         host_words.close()
         dev_words.close()
         flag.close()
+
+
+@pytest.mark.parametrize("pool", [PinnedBuffer, DeviceBuffer])
+def test_layers_of_zero_byte_blocks_are_marked(gpu, pool):
+    """A layout that says its blocks hold no bytes: nothing moves, every word is set."""
+    say(f"[gpu] marks of layers without bytes, {pool.__name__}")
+    dev, host, words = DeviceBuffer(4096), pool(4096), PinnedBuffer(16)
+    words.array[:] = 0
+    reg = KVCacheRegistration.create(dev.ptr, 4096, 16, 256, 0, 1)
+    reg = dataclasses.replace(reg, block_size_bytes=0)
+    x = TransferContext(0)
+    try:
+        layer = LayerTransfer(reg, block_array([1, 2], [host.ptr, host.ptr + 256]))
+        x.load_layers_marked([layer, layer], [(words.ptr, 7, True)], _lib.MODE_KERNEL)
+        x.synchronize()
+        assert words.array.view(np.uint64).tolist() == [7, 7]
+    finally:
+        x.close()
+        for b in (dev, host, words):
+            b.close()
 
 
 class MarkedCopies:
