@@ -474,7 +474,9 @@ int pf_save_layers(pf_xfer* xfer, const pf_layer_xfer* layers,
  * are in place (per-layer completion, which the reference lacks:
  * worker.py:288-289).  Completion of the whole call is pf_xfer_synchronize or
  * the last layer's event.  A save or load that fails returns with none of
- * its copies (or marks) still in flight. */
+ * its copies (or marks) still in flight.  One that is refused for what its
+ * arguments say has moved nothing, but for a large call over the host link,
+ * whose first layers are under way before the others are checked. */
 int pf_load_layers(pf_xfer* xfer, const pf_layer_xfer* layers,
                    uint32_t num_layers, uint32_t mode, pf_event* layer_events);
 

@@ -234,6 +234,8 @@ int engine_signal_wait(EngineSignal* s, bool spin = false);
 class RangeCache {
  public:
   bool check(uint64_t addr, uint64_t len);
+  // check, with the bounds of the allocation.
+  bool find(uint64_t addr, uint64_t len, uint64_t* begin, uint64_t* end);
 
  private:
   bool contains(uint64_t addr, uint64_t len);

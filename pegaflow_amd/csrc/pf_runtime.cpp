@@ -111,6 +111,13 @@ bool RangeCache::check(uint64_t a, uint64_t len) {
   return true;
 }
 
+bool RangeCache::find(uint64_t a, uint64_t len, uint64_t* begin, uint64_t* end) {
+  if (!check(a, len)) return false;
+  *begin = last_b_;
+  *end = last_e_;
+  return true;
+}
+
 static int check_range(uint64_t addr, uint64_t len, const char* what) {
   RangeCache rc;
   if (!rc.check(addr, len))

@@ -3,10 +3,12 @@
 // copy loops of gpu_worker.rs with gather/scatter kernels.
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <deque>
+#include <functional>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -204,25 +206,43 @@ void gathered(const ChunkList& a, LayerPlan* p) {
   p->host_increasing = a.increasing;
 }
 
-// The usual layer in one pass over its blocks: a split layout, or whole blocks,
-// with every block in bounds and every host address given.  False when some
-// block is not: plan_layer then goes through the checks one by one for the
-// reference's error.  One pass instead of one per check, here and in the calls'
-// later checks: 40,960 chunks of a gather between device buffers, 585 -> 520 us
-// a call with the Python layer's marshalling.
+// The chunks of the usual layer, a split layout or whole blocks: their size, and
+// the blocks up to max_block (none unless `any`) that have theirs in bounds.
+struct LayerBounds {
+  bool split = false, any = false;
+  uint64_t bytes = 0, v_off = 0, max_block = 0;
+};
+
+LayerBounds layer_bounds(const pf_kv_layout& l, bool split) {
+  const uint64_t seg = l.bytes_per_block;
+  LayerBounds b;
+  b.split = split;
+  b.bytes = split ? seg : l.block_size_bytes;
+  const SegBound k = seg_bound(l, 0, b.bytes >= seg ? b.bytes : seg);
+  const SegBound v = split ? seg_bound(l, 1, seg) : k;
+  b.any = k.any && v.any;
+  b.v_off = v.seg_off;
+  b.max_block = std::min(k.max_block, v.max_block);
+  return b;
+}
+
+// The usual layer in one pass over its blocks, with every block in bounds and
+// every host address given.  False when some block is not: plan_layer then goes
+// through the checks one by one for the reference's error.  One pass instead of
+// one per check, here and in the calls' later checks: 40,960 chunks of a gather
+// between device buffers, 585 -> 520 us a call with the Python layer's
+// marshalling.
 bool plan_in_bounds(const pf_layer_xfer& lx, bool split, LayerPlan* out) {
   const pf_kv_layout& l = lx.layout;
   const uint64_t seg = l.bytes_per_block;
   const size_t n = static_cast<size_t>(lx.num_blocks);
-  const uint64_t bytes = split ? seg : l.block_size_bytes;
-  const SegBound k = seg_bound(l, 0, bytes >= seg ? bytes : seg);
-  const SegBound v = split ? seg_bound(l, 1, seg) : k;
-  if (n == 0 || !k.any || !v.any) return false;
-  const uint64_t max_block = std::min(k.max_block, v.max_block);
+  const LayerBounds bounds = layer_bounds(l, split);
+  const uint64_t bytes = bounds.bytes, max_block = bounds.max_block;
+  if (n == 0 || !bounds.any) return false;
   out->chunk_bytes = bytes;
   out->chunks.resize(split ? 2 * n : n);
   ChunkList kl{out->chunks.data(), bytes}, vl{out->chunks.data() + n, bytes};
-  const uint64_t v_at = l.data_ptr + v.seg_off;
+  const uint64_t v_at = l.data_ptr + bounds.v_off;
   uint64_t top = 0;
   bool host = true;
   if (split) {
@@ -486,6 +506,8 @@ struct pf_xfer {
   // capacity for the next call: a call plans tens of thousands of chunks,
   // and fresh buffers each time cost page faults before the first launch.
   std::vector<LayerPlan> plans, plans_rest;
+  // Allocations that the call in progress (under mu) has found.
+  RangeCache ranges;
   std::mutex mu;
 };
 
@@ -799,9 +821,8 @@ int plan_all(const pf_layer_xfer* layers, uint32_t n, bool is_save,
   return PF_OK;
 }
 
-int check_all_kernel(const pf_layer_xfer* layers, const std::vector<LayerPlan>& plans,
-                     bool host_side) {
-  RangeCache rc;
+int check_all_kernel(RangeCache& rc, const pf_layer_xfer* layers,
+                     const std::vector<LayerPlan>& plans, bool host_side) {
   for (size_t i = 0; i < plans.size(); ++i) {
     if (plans[i].chunks.empty() || plans[i].ordered) continue;
     if (int r = check_device_tensor(rc, layers[i].layout)) return r;
@@ -1011,7 +1032,8 @@ struct PinnedCache {
 // waited for before the next is queued.
 int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<LayerPlan>& plans,
                   bool is_save, pf_event* layer_events, const SignalTargets* sig,
-                  bool wait_save, size_t desc_off, uint32_t layer_base, size_t* used);
+                  bool wait_save, size_t desc_off, uint32_t layer_base, size_t* used,
+                  const std::function<bool()>& sure = {});
 
 int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
                   std::vector<LayerPlan>& plans, StagedPlanner& planner, StagedPlan& sp,
@@ -1381,7 +1403,8 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
   return PF_OK;
 }
 
-uint32_t pipeline_head(const pf_layer_xfer* layers, uint32_t num_layers);
+uint32_t pipeline_head(const pf_layer_xfer* layers, uint32_t num_layers,
+                       bool* device_copy = nullptr);
 
 // A staged call.  `pending`: layers from pending->head on are listed once
 // pending->ready() returns.
@@ -1615,6 +1638,8 @@ bool host_side_pinned(const LayerPlan& p) {
 bool host_sourced(const LayerPlan& p, bool is_save) { return !is_save && host_side_pinned(p); }
 
 // ---- kernel mode ----------------------------------------------------------
+constexpr int kNotSure = INT_MIN;  // kernel_direct's, never a call's result
+
 // One step of a kernel-mode call: a DMA copy of an ordered layer, or one
 // launch over the consecutive layers [li, lj).
 struct Step {
@@ -1632,13 +1657,14 @@ struct Step {
 // index of plans[0] (marks and their counters are per call-wide layer).
 // *used (if given): the descriptor slots of d_desc from desc_off on that
 // this call's launches read (chunks, then the marks' tables), 0 when they
-// read in place.
+// read in place.  sure (if given): asked before the first copy; kNotSure when it
+// says no.
 int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<LayerPlan>& plans,
                   bool is_save, pf_event* layer_events, const SignalTargets* sig,
                   bool wait_save, size_t desc_off = 0, uint32_t layer_base = 0,
-                  size_t* used = nullptr) {
+                  size_t* used = nullptr, const std::function<bool()>& sure) {
   if (used) *used = 0;
-  if (int rc = check_all_kernel(layers, plans, true)) return rc;
+  if (int rc = check_all_kernel(x->ranges, layers, plans, true)) return rc;
   size_t total = 0;
   std::vector<size_t> first(plans.size());
   for (size_t li = 0; li < plans.size(); ++li) {
@@ -1735,6 +1761,7 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     if (int rc = upload_desc(x, total + aux_desc, desc_off)) return rc;
     if (used) *used = total + aux_desc;
   }
+  if (sure && !sure()) return kNotSure;
   const uint32_t* d_aux = reinterpret_cast<const uint32_t*>(x->desc_base + total);
   for (const Step& st : steps) {
     if (st.dma) {
@@ -1818,7 +1845,54 @@ uint32_t pf::pipeline_head_layers(uint32_t num_layers, uint64_t chunks) {
 
 namespace {
 
-uint32_t pipeline_head(const pf_layer_xfer* layers, uint32_t num_layers) {
+// Layers [begin, end) are sure to pass the checks that planning and issuing them
+// make (false: they may not, or a block leaves its V address to be derived).  A
+// copy between device buffers is issued in parts only then, so that one that is
+// refused has moved nothing.
+//
+// Per layer, all addresses in one allocation, known from the first.  One pass of
+// differences whose signs are gathered (addresses and sizes are below 2^63), under
+// the upload of the first part's descriptors: of a Llama prefix's gather 2 us where
+// the layers share an allocation (478 -> 480), 11 where each is one of its own (472
+// -> 483), since their allocations are looked up before the first copy.
+bool layers_sure(RangeCache& rc, const pf_layer_xfer* layers, uint32_t begin, uint32_t end,
+                 bool is_save) {
+  for (uint32_t li = begin; li < end; ++li) {
+    const pf_layer_xfer& lx = layers[li];
+    const pf_kv_layout& l = lx.layout;
+    if (l.bytes_per_block == 0 || l.segments == 0 || l.num_blocks == 0) return false;
+    if (lx.num_blocks == 0) continue;
+    const int kind = layout_kind(l);
+    if (!lx.blocks || (kind == PF_LAYOUT_STRIDED && is_save)) return false;
+    const LayerBounds bounds = layer_bounds(l, kind == PF_LAYOUT_SPLIT);
+    uint64_t lo = 0, hi = 0;
+    if (!bounds.any || bounds.bytes / 16 >= (1ull << 31) || (bounds.max_block >> 63) != 0 ||
+        !rc.check(l.data_ptr, l.size_bytes) ||
+        !rc.find(lx.blocks[0].k_host, bounds.bytes, &lo, &hi) || (hi >> 63) != 0)
+      return false;
+    const uint64_t room = hi - lo - bounds.bytes;  // of a chunk's first byte from lo
+    uint64_t bad = 0;
+    auto inside = [&](uint64_t v, uint64_t most) { bad |= v | (most - v); };
+    if (bounds.split) {
+      for (uint64_t i = 0; i < lx.num_blocks; ++i) {
+        const pf_block_xfer& b = lx.blocks[i];
+        inside(static_cast<uint64_t>(b.block_idx), bounds.max_block);
+        inside(b.k_host - lo, room);
+        inside(b.v_host - lo, room);
+      }
+    } else {
+      for (uint64_t i = 0; i < lx.num_blocks; ++i) {
+        const pf_block_xfer& b = lx.blocks[i];
+        inside(static_cast<uint64_t>(b.block_idx), bounds.max_block);
+        inside(b.k_host - lo, room);
+      }
+    }
+    if (bad >> 63) return false;
+  }
+  return true;
+}
+
+uint32_t pipeline_head(const pf_layer_xfer* layers, uint32_t num_layers, bool* device_copy) {
   if (num_layers < 8) return 0;
   uint64_t chunks = 0;
   const pf_block_xfer* first = nullptr;
@@ -1829,14 +1903,18 @@ uint32_t pipeline_head(const pf_layer_xfer* layers, uint32_t num_layers) {
   uint64_t b = 0, e = 0;
   if (!first) return 0;
   const uint32_t head = pipeline_head_layers(num_layers, chunks);
-  return head > 0 && !pinned_lookup(first->k_host, 1, &b, &e) ? num_layers / 4 : head;
+  if (head == 0 || pinned_lookup(first->k_host, 1, &b, &e)) return head;
+  if (device_copy) *device_copy = true;
+  return num_layers / 4;
 }
 
 // pending: the layers from `head` on are filled in by pending->ready(),
-// called once the first part is issued.
+// called once the first part is issued.  device_copy: kNotSure, with no copy
+// issued, when the layers from `head` on may be refused.
 int kernel_pipelined(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
-                     uint32_t head, bool is_save, bool wait_save, const SignalTargets* sig,
-                     pf_event* layer_events, const PendingLayers* pending = nullptr) {
+                     uint32_t head, bool device_copy, bool is_save, bool wait_save,
+                     const SignalTargets* sig, pf_event* layer_events,
+                     const PendingLayers* pending = nullptr) {
   std::vector<LayerPlan>& first = x->plans;
   std::vector<LayerPlan>& rest = x->plans_rest;
   if (int rc = plan_all(layers, head, is_save, &first)) return rc;
@@ -1855,12 +1933,15 @@ int kernel_pipelined(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layer
   // The second part's descriptors go after everything the first part's
   // launches read: its chunks and its mark tables.
   size_t n_first = 0;
-  if (int rc = kernel_direct(x, layers, first, is_save, layer_events, sig, false, 0, 0,
-                             &n_first))
-    return rc;
-  if (pending)
+  auto sure = [&] { return layers_sure(x->ranges, layers, head, num_layers, is_save); };
+  int rc = kernel_direct(x, layers, first, is_save, layer_events, sig, false, 0, 0, &n_first,
+                         device_copy ? std::function<bool()>(sure) : nullptr);
+  if (rc != PF_OK) return rc;
+  if (pending) {
     if (int rc = pending->ready()) return rc;
-  int rc = plan_all(layers + head, num_layers - head, is_save, &rest);
+    x->ranges = RangeCache();  // the caller has run meanwhile
+  }
+  rc = plan_all(layers + head, num_layers - head, is_save, &rest);
   if (rc == PF_OK) {
     for (uint32_t li = head; li < num_layers; ++li)
       apply_write_policy(layers[li], is_save, false, &rest[li - head]);
@@ -1886,6 +1967,7 @@ int run(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers, uint32_t m
   std::lock_guard<std::mutex> lk(x->mu);
   x->last_kernels = 0;
   x->last_dma = 0;
+  x->ranges = RangeCache();
   PF_HIP(hipSetDevice(x->device));
   const int rc =
       run_locked(x, layers, num_layers, mode, is_save, layer_events, wait_save, sig, pending);
@@ -1953,11 +2035,15 @@ int run_locked(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers, uin
     // rest are planned, so the planning of the rest (about 3 ns a chunk)
     // overlaps their copy.  Marks carry call-wide layer indices; per-layer
     // events stay with their layers.
-    const uint32_t head = pending ? pending->head : pipeline_head(layers, num_layers);
-    if (head > 0 && head < num_layers)
-      return kernel_pipelined(x, layers, num_layers, head, is_save, wait_save,
-                              is_save ? nullptr : sig, is_save ? nullptr : layer_events,
-                              pending);
+    bool device_copy = false;
+    const uint32_t head =
+        pending ? pending->head : pipeline_head(layers, num_layers, &device_copy);
+    if (head > 0 && head < num_layers) {
+      const int rc =
+          kernel_pipelined(x, layers, num_layers, head, device_copy, is_save, wait_save,
+                           is_save ? nullptr : sig, is_save ? nullptr : layer_events, pending);
+      if (rc != kNotSure) return rc;
+    }
   }
   if (mode == PF_MODE_STAGED)
     return staged(x, layers, num_layers, is_save, layer_events, sig, wait_save, pending);

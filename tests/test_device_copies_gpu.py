@@ -204,6 +204,43 @@ def test_more_workgroups_than_tiles(gpu, n):
     ctx.close()
 
 
+# What a call is refused for in its last layer: a block past the tensor, one below it,
+# no address for a block, an address in no allocation.
+@pytest.mark.parametrize("bad", [("block_idx", 600), ("block_idx", -1), ("k_host", 0),
+                                 ("k_host", 4096), ("v_host", 4096)])
+def test_refused_device_copy_moves_nothing(gpu, bad):
+    """Copies between device buffers of enough chunks to be issued in parts (16 layers of
+    512 blocks), with the last layer at fault; without the fault they run."""
+    layers = make_layers(np.random.default_rng(5), 256, 2, (512,) * 16, 600)
+    pool = DeviceBuffer(sum(l.nbytes for l in layers))
+    ctx = TransferContext(0)
+    for ok in (False, True):
+        xfers = [l.transfer(b) for l, b in zip(layers, bases(layers, pool.ptr))]
+        if not ok:
+            xfers[-1].blocks[bad[0]][511] = bad[1]
+        pool.memset(0xa5)
+        if ok:
+            ctx.save_layers(xfers, _lib.MODE_KERNEL)
+            assert np.array_equal(pool.download(), np.concatenate([l.packed() for l in layers]))
+        else:
+            with pytest.raises(_lib.PegaFlowError):
+                ctx.save_layers(xfers, _lib.MODE_KERNEL)
+            assert (pool.download() == 0xa5).all()
+        pool.fill_random(7)
+        packed = pool.download()
+        if ok:
+            ctx.load_layers(xfers, _lib.MODE_KERNEL)
+        else:
+            with pytest.raises(_lib.PegaFlowError):
+                ctx.load_layers(xfers, _lib.MODE_KERNEL)
+        ctx.synchronize()
+        for l, at in zip(layers, bases(layers, 0)):
+            if ok:
+                l.restore(packed[at:at + l.nbytes])
+            assert np.array_equal(l.dev.download(), l.host)
+    ctx.close()
+
+
 # Chunks shorter than a word, around one, around a unit, and of several units, at
 # every kind of offset from a word's boundary.
 UNALIGNED = [(bpb, off) for bpb in (1, 7, 15, 16, 17, 33, 200, 1009, 1023, 1025, 1041, 2060, 12301)
