@@ -687,7 +687,7 @@ int check_launch_size(size_t n, uint64_t chunk_bytes) {
 
 int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, bool is_save,
            bool host_side = false, const LayerMarks* marks = nullptr,
-           hipStream_t stream = nullptr) {
+           hipStream_t stream = nullptr, bool first_part = false) {
   if (n == 0) return PF_OK;
   if (!stream) stream = x->stream;
   const int dir = (is_save ? PF_ROUTE_SAVE_DEVICE : PF_ROUTE_LOAD_DEVICE) + (host_side ? 2 : 0);
@@ -716,7 +716,10 @@ int launch(pf_xfer* x, size_t first, size_t n, uint64_t chunk_bytes, bool al16, 
   uint32_t threads = x->threads[dir], unroll = x->unroll[dir];
   ScatterTrial* trial = nullptr;
   if ((unroll & PF_KERNEL_AUTO) && dir == PF_ROUTE_LOAD_DEVICE && al16 && qgrid == 0) {
-    const int pick = scatter_pick(x, static_cast<uint64_t>(n) * chunk_bytes, &trial);
+    // The first part of a call in two has a third of the other's bytes, and its
+    // fixed costs three times the weight: it is not timed.
+    const int pick =
+        scatter_pick(x, first_part ? 0 : static_cast<uint64_t>(n) * chunk_bytes, &trial);
     threads = kScatterShapes[pick][0];
     unroll = kScatterShapes[pick][1];
     if (trial) PF_HIP(hipEventRecord(trial->start, stream));
@@ -1657,8 +1660,8 @@ struct Step {
 // index of plans[0] (marks and their counters are per call-wide layer).
 // *used (if given): the descriptor slots of d_desc from desc_off on that
 // this call's launches read (chunks, then the marks' tables), 0 when they
-// read in place.  sure (if given): asked before the first copy; kNotSure when it
-// says no.
+// read in place.  sure (given for the first part of a copy between device
+// buffers): asked before the first copy; kNotSure when it says no.
 int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<LayerPlan>& plans,
                   bool is_save, pf_event* layer_events, const SignalTargets* sig,
                   bool wait_save, size_t desc_off = 0, uint32_t layer_base = 0,
@@ -1806,7 +1809,7 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
           break;
         }
       if (int rc = launch(x, first[st.li], n, plans[st.li].chunk_bytes, st.aligned, is_save,
-                          host_side, marked ? &marks : nullptr))
+                          host_side, marked ? &marks : nullptr, nullptr, sure != nullptr))
         return rc;
     }
     if (layer_events && layer_events[st.li])

@@ -241,6 +241,31 @@ def test_refused_device_copy_moves_nothing(gpu, bad):
     ctx.close()
 
 
+# 16 layers, of which the first 4 are a part of their own: the bytes and blocks of those
+# and of the others, and whether the others are large enough to be timed.
+@pytest.mark.parametrize("first,rest,timed", [((32768, 512), (256, 1024), False),
+                                              ((256, 64), (32768, 700), True)])
+def test_scatter_trials_time_no_first_part(gpu, first, rest, timed):
+    """The scatter's two shapes are compared on launches that are not a call's first part,
+    whose share of the call, and so of its fixed costs, is another."""
+    rng = np.random.default_rng(3)
+    layers = [layer for bpb, n in (first,) * 4 + (rest,) * 12
+              for layer in make_layers(rng, bpb, 2, (n,), n + 3)]
+    pool = DeviceBuffer(sum(l.nbytes for l in layers))
+    pool.fill_random(9)
+    packed = pool.download()
+    ctx = TransferContext(0)
+    for _ in range(4):
+        ctx.load_layers([l.transfer(b) for l, b in zip(layers, bases(layers, pool.ptr))],
+                        _lib.MODE_KERNEL)
+        ctx.synchronize()
+    assert ctx.route_shape(_lib.ROUTE_LOAD_DEVICE)[2] is timed
+    for l, at in zip(layers, bases(layers, 0)):
+        l.restore(packed[at:at + l.nbytes])
+        assert np.array_equal(l.dev.download(), l.host)
+    ctx.close()
+
+
 # Chunks shorter than a word, around one, around a unit, and of several units, at
 # every kind of offset from a word's boundary.
 UNALIGNED = [(bpb, off) for bpb in (1, 7, 15, 16, 17, 33, 200, 1009, 1023, 1025, 1041, 2060, 12301)
