@@ -25,6 +25,15 @@ inline bool table_in_place(size_t n, uint64_t chunk_bytes, bool is_save) {
   return n <= kQueueTableMax && !(is_save && n > 512 && chunk_bytes < 4096);
 }
 
+// Whether a call of n descriptors leaves them in host memory for the waves of a
+// copy between device buffers, which read their own: `narrow` bytes of its copies
+// go by waves of 1 KiB, a read each.  In place less uploaded, us a call: 1,024
+// chunks of 32 KiB gather -3.5, of 64 KiB -1.3, of 128 KiB +1.4, of 256 KiB +7.1,
+// of 512 KiB +13.4 (and scattered by waves of 2 KiB, or marked, -3 to -10 all the
+// way); of 64 KiB and 3 bytes -0.3, of 128 KiB and 3 bytes +6.  The waves of one
+// chunk share its read, so few chunks cost little: 32 of 8 MiB -5.5.
+inline bool waves_in_place(size_t n, uint64_t narrow) { return n <= 64 || narrow <= 64ull << 20; }
+
 // Workgroups of a load of n chunks in place on a route at its default grid.  Each
 // reads the whole table first, and a load of few bytes has no work for many:
 // with 16 and 64 workgroups, 2 MiB (64 chunks of 32 KiB) load in 61.7 and 65.3 us,

@@ -670,6 +670,15 @@ int scatter_pick(pf_xfer* x, uint64_t bytes, ScatterTrial** timed) {
   return i;
 }
 
+// Loads in flight per lane of the next fixed-map launch of aligned chunks between
+// device buffers (0: such launches are queued).
+uint32_t fixed_unroll(const pf_xfer* x, bool is_save) {
+  const uint32_t route = is_save ? PF_ROUTE_SAVE_DEVICE : PF_ROUTE_LOAD_DEVICE;
+  if (x->grid[route] > 0) return 0;
+  const bool chosen = (x->unroll[route] & PF_KERNEL_AUTO) && route == PF_ROUTE_LOAD_DEVICE;
+  return (chosen ? kScatterShapes[std::max(x->scatter_choice, 0)][1] : x->unroll[route]) & 0xffu;
+}
+
 void scatter_trials_reset(pf_xfer* x) {
   x->scatter_choice = -1;
   for (ScatterTrial& t : x->trials) {
@@ -1669,10 +1678,13 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
   if (used) *used = 0;
   if (int rc = check_all_kernel(x->ranges, layers, plans, true)) return rc;
   size_t total = 0;
+  uint64_t bytes = 0;
   std::vector<size_t> first(plans.size());
   for (size_t li = 0; li < plans.size(); ++li) {
     first[li] = total;
-    if (!plans[li].ordered) total += plans[li].chunks.size();
+    if (plans[li].ordered) continue;
+    total += plans[li].chunks.size();
+    bytes += plans[li].chunks.size() * plans[li].chunk_bytes;
   }
   // Without per-layer events, consecutive layers with the same chunk size and
   // alignment share one launch (marks keep per-layer completion inside it).
@@ -1735,11 +1747,22 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
   // Counters for marks and the tile queue of queued launches.
   if (int rc = ensure_counters(x, layer_base + plans.size())) return rc;
   ChunkDesc* hd = desc_off ? nullptr : small_desc(x, total + aux_desc);
-  // Host-side launches are queued, and take the whole table into LDS.
-  if (hd && total > 0)
-    for (const LayerPlan& p : plans)
-      if (!p.ordered && !table_in_place(total, p.chunk_bytes, is_save) && host_side_pinned(p))
-        hd = nullptr;
+  if (hd) {
+    // Host-side launches are queued, and take the whole table into LDS; the waves
+    // of a fixed map read their own descriptor (marked copies' move 2 KiB each).
+    const uint32_t unroll = fixed_unroll(x, is_save);
+    const bool all_in_place = waves_in_place(total, bytes);
+    uint64_t narrow = 0;
+    for (const LayerPlan& p : plans) {
+      if (p.ordered || p.chunks.empty()) continue;
+      const bool table = table_in_place(total, p.chunk_bytes, is_save);
+      const bool wide = sig || all_in_place || (unroll != 1 && chunks_aligned(p));
+      if (table && wide) continue;
+      if (!host_side_pinned(p)) narrow += wide ? 0 : p.chunks.size() * p.chunk_bytes;
+      else if (!table) hd = nullptr;
+    }
+    if (!waves_in_place(total, narrow)) hd = nullptr;
+  }
   if (desc_off) {
     if (desc_off + total + aux_desc > x->h_cap || desc_off + total + aux_desc > x->d_cap)
       return fail(PF_ERR_INVALID_ARGUMENT, "descriptor room not reserved");

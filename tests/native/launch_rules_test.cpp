@@ -2,7 +2,8 @@
 // (no GPU), built by tests/test_native.py from the library's own sources:
 //   * a queued launch keeps its route's workgroups, loads in flight and flags;
 //   * a small load at the default grid: workgroups by its bytes;
-//   * the calls over the host link whose descriptors are read in place;
+//   * the calls over the host link, and between device buffers, whose
+//     descriptors are read in place;
 //   * chunks smaller than a tile: workgroups of the chunk's size, as many
 //     lanes in all, within the caps.
 // Exit status 0 and "ok" on success; the first failed checks are printed.
@@ -62,6 +63,12 @@ int main() {
     expect(table_in_place(513, 4080, is_save) == !is_save, what + ", short chunks");
     expect(!table_in_place(1025, 4096, is_save), what + ", many chunks");
   }
+  // Between device buffers: by the bytes that waves of 1 KiB move, but for few chunks.
+  const uint64_t MiB = 1ull << 20;
+  expect(waves_in_place(2048, 64 * MiB) && waves_in_place(65, 0), "narrow waves in place");
+  expect(!waves_in_place(2048, 64 * MiB + 1) && !waves_in_place(65, 512 * MiB),
+         "narrow waves uploaded");
+  expect(waves_in_place(64, 512 * MiB) && waves_in_place(1, 1ull << 40), "few chunks in place");
   if (failures) {
     std::printf("%d checks failed\n", failures);
     return 1;
