@@ -369,11 +369,10 @@ int pf_xfer_route_shape(pf_xfer* xfer, uint32_t route, uint32_t* threads,
  * a marked load's layers, finishing in order, and few requests in flight
  * keep the link at its peak).  Marked launches out of pinned host memory
  * always run queued (at PF_LOAD_HOST_DEFAULT_GRID when their route says 0);
- * marked copies between device buffers have a workgroup per up to 8 or 32 KiB
- * of a layer.  A
- * load of up to 1,024 chunks and 8 MiB on a route at PF_LOAD_HOST_DEFAULT_GRID
- * runs with one workgroup a 128 KiB, at least 16; any other setting holds as it
- * is.  pf_xfer_set_max_grid caps both kinds.  Every route may run queued: the
+ * marked copies between device buffers have a workgroup per up to 8, 32 or 64
+ * KiB of a layer.  A load of up to 1,024 chunks and 8 MiB on a route at
+ * PF_LOAD_HOST_DEFAULT_GRID runs with one workgroup a 128 KiB, at least 16; any
+ * other setting holds as it is.  pf_xfer_set_max_grid caps both kinds.  Every route may run queued: the
  * staged mode's two streams each have a queue of their own, and a queued launch
  * leaves its queue empty. */
 #define PF_SAVE_HOST_DEFAULT_GRID 32u

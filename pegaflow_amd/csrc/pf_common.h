@@ -82,11 +82,20 @@ struct MarkedShape {
   uint32_t units_per_chunk;
   uint32_t wg_units;  // units of one workgroup
 };
-inline MarkedShape marked_shape(uint64_t chunk_bytes, uint64_t launch_chunks, bool aligned) {
+inline MarkedShape marked_shape(uint64_t chunk_bytes, uint64_t launch_chunks,
+                                uint64_t launch_layers, bool aligned) {
   const uint64_t unit = 64ull * 16 * (aligned ? kMarkedUnroll : 1);
-  // Up to 32 KiB a workgroup, and 8 KiB in launches too small to fill the chip
-  // with those (see copy_chunks_marked_kernel).
-  const uint64_t share = launch_chunks * chunk_bytes >= (32ull << 20) ? 32768 : 8192;
+  // Bytes of a workgroup, at most: each adds to its layer's counter, one after
+  // another, so large layers take large shares, and launches too small to fill the
+  // chip with those take small ones.  Kernel times with shares of 8, 32 and 64 KiB,
+  // us: one layer of 4 MiB 13.4, 10.0 and 10.8, of 10 MiB 22.6, 12.9 and 11.9, of
+  // 40 MiB 67, 27.7 and 21.8 (128 KiB 24.5); 8 of 40 MiB 325, 125 and 118; 32 of 2
+  // MiB 33, 21.3 and 21.4; 61 of 4.7 MB 129, 93.0 and 94.5.
+  const uint64_t bytes = launch_chunks * chunk_bytes;
+  const uint64_t layer = bytes / (launch_layers ? launch_layers : 1);
+  const uint64_t share = layer >= (16ull << 20)                             ? 65536
+                         : bytes >= (32ull << 20) || layer >= (2ull << 20) ? 32768
+                                                                            : 8192;
   // An unaligned chunk's words lie between its first and last few bytes, and a
   // chunk of those only still has a unit.
   const uint64_t units = aligned ? (chunk_bytes + unit - 1) / unit
@@ -152,8 +161,8 @@ hipError_t launch_copy_chunks_queue(const ChunkDesc* d_descs, uint32_t n_chunks,
                                     uint32_t* queue, hipStream_t stream);
 // A marked copy between device buffers: each finished layer of the marks is
 // marked.  At most max_grid workgroups (0: no cap).  The table's n_wg workgroups
-// and its entries are those of marked_shape(chunk_bytes, n_chunks, aligned16) over
-// its layers; marks by value need 16-byte aligned chunks.
+// and its entries are those of marked_shape(chunk_bytes, n_chunks, n, aligned16)
+// over its n layers; marks by value need 16-byte aligned chunks.
 hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks,
                                      uint64_t chunk_bytes, uint32_t max_grid, SliceMarks marks,
                                      hipStream_t stream);

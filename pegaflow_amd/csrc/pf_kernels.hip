@@ -232,9 +232,8 @@ __device__ __forceinline__ void copy_unaligned_unit(const ChunkDesc& d, uint32_t
 // Bound by HBM and by the reports.  A unit is 64 lanes x UNROLL words of one
 // chunk and belongs to one wave, so a chunk of any size wastes at most part of
 // its last unit.  Workgroup w copies the consecutive units of one layer that
-// its index gives it and then adds their number to the layer's counter, once:
-// adds to one counter run one after another (about 40 ns): one per 4 KiB doubled
-// the time of the whole copy, one per 32 KiB costs 0-5% of it.
+// its index gives it (see marked_shape) and then adds their number to the layer's
+// counter, once: adds to one counter run one after another (about 20 ns).
 // Workgroups start in index order, so the layers land in order.
 //
 // Visibility: as in the marking protocol above, with 16-byte write-through
@@ -242,9 +241,8 @@ __device__ __forceinline__ void copy_unaligned_unit(const ChunkDesc& d, uint32_t
 // us, ordinary 97, non-temporal 105-115), so no L2 has to be written back
 // before a report.  The per-workgroup release fence that this replaces allowed
 // only 128 workgroups.  61 layers of 4.7 MB, one launch and one marking kernel
-// each before, took 450 us, here 94 in one launch.  A launch of a single 40 MiB
-// layer (a staged slice, under the next slice's copy) is bound by its 1,280 adds
-// to one counter: 28.7 us, where 128 workgroups with fences took 24.0.
+// each before, took 450 us, here 94 in one launch; a single 40 MiB layer (a staged
+// slice, under the next slice's copy) takes 21.8, with the fences 24.0.
 //
 // Chunks that are not aligned (ALIGNED false) go by units of 64 words, their odd
 // bytes written through as well: 61 layers of 4.7 MB in 36,865-byte chunks land
@@ -741,7 +739,7 @@ hipError_t launch_copy_chunks_marked(const ChunkDesc* d_descs, uint32_t n_chunks
       marks.targets.count == 0 || marks.targets.count > kMaxSignalTargets ||
       marks.chunk_start[0] != 0 || marks.chunk_start[marks.n] != n_chunks)
     return hipErrorInvalidValue;
-  const MarkedShape s = marked_shape(chunk_bytes, n_chunks, true);
+  const MarkedShape s = marked_shape(chunk_bytes, n_chunks, marks.n, true);
   // Groups in chunk order, each counting at least its own units.
   uint64_t wg = 0;
   for (uint32_t g = 0; g < marks.n; ++g) {
@@ -766,7 +764,7 @@ hipError_t launch_copy_chunks_mark_table(const ChunkDesc* d_descs, uint32_t n_ch
   if (marks.n == 0 || !marks.wg_start || !marks.chunk_start || !marks.layer || !marks.counters ||
       marks.targets.count == 0 || marks.targets.count > kMaxSignalTargets)
     return hipErrorInvalidValue;
-  const MarkedShape s = marked_shape(chunk_bytes, n_chunks, aligned16);
+  const MarkedShape s = marked_shape(chunk_bytes, n_chunks, marks.n, aligned16);
   if (!marked_fits(s, n_chunks, chunk_bytes, aligned16, n_wg)) return hipErrorInvalidValue;
   return aligned16 ? launch_marked<true>(d_descs, chunk_bytes, s, n_wg, max_grid, marks, stream)
                    : launch_marked<false>(d_descs, chunk_bytes, s, n_wg, max_grid, marks, stream);

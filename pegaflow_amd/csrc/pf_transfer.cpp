@@ -1240,7 +1240,7 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
         m.chunk_start[m.n + 1] = m.chunk_start[m.n] + static_cast<uint32_t>(pc.end - pc.begin);
         if (self_marked[pc.layer] == 1) {
           m.units[m.n] = static_cast<uint32_t>(
-              p.chunks.size() * marked_shape(p.chunk_bytes, st.n_chunks, true).units_per_chunk);
+              p.chunks.size() * marked_shape(p.chunk_bytes, st.n_chunks, 1, true).units_per_chunk);
           counts = true;
         }
         ++m.n;
@@ -1715,9 +1715,12 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     Step st{li, lj, false, al};
     if (sig && (al || !host_src) && p.chunk_bytes > 0 && !layer_events) {
       st.tab = aux.size();
-      size_t chunks = 0;
-      for (size_t k = li; k < lj; ++k) chunks += plans[k].chunks.size();
-      const MarkedShape shape = marked_shape(p.chunk_bytes, chunks, al);
+      size_t chunks = 0, groups = 0;
+      for (size_t k = li; k < lj; ++k) {
+        chunks += plans[k].chunks.size();
+        groups += !plans[k].chunks.empty();
+      }
+      const MarkedShape shape = marked_shape(p.chunk_bytes, chunks, groups, al);
       std::vector<uint32_t> ids, wg_start;
       uint64_t start = 0, wgs = 0;
       for (size_t k = li; k < lj; ++k) {

@@ -4,6 +4,7 @@
 //   * a small load at the default grid: workgroups by its bytes;
 //   * the calls over the host link, and between device buffers, whose
 //     descriptors are read in place;
+//   * a marked copy's workgroups a layer, by the layer's and the launch's bytes;
 //   * chunks smaller than a tile: workgroups of the chunk's size, as many
 //     lanes in all, within the caps.
 // Exit status 0 and "ok" on success; the first failed checks are printed.
@@ -69,6 +70,23 @@ int main() {
   expect(!waves_in_place(2048, 64 * MiB + 1) && !waves_in_place(65, 512 * MiB),
          "narrow waves uploaded");
   expect(waves_in_place(64, 512 * MiB) && waves_in_place(1, 1ull << 40), "few chunks in place");
+  // Workgroups that report a layer of a marked copy, one after another: few enough
+  // for large layers, and enough of them in launches of small ones.
+  const uint64_t marked[][4] = {{1280, 32768, 1, 640},  {640, 32768, 1, 320},
+                                {128, 32768, 1, 128},   {32, 32768, 1, 128},
+                                {10240, 32768, 8, 640}, {7808, 36864, 61, 144},
+                                {64, 32768, 32, 8}};
+  for (const auto& t : marked) {
+    const MarkedShape s = marked_shape(t[1], t[0], t[2], true);
+    expect(marked_workgroups(s, t[0] / t[2]) == t[3],
+           "marked copy of " + std::to_string(t[0]) + " chunks in " + std::to_string(t[2]) +
+               " layers: " + std::to_string(marked_workgroups(s, t[0] / t[2])));
+    // The units of a chunk do not depend on the launch that copies it.
+    expect(s.units_per_chunk == marked_shape(t[1], 1, 1, true).units_per_chunk, "units");
+  }
+  const uint64_t odd[][2] = {{1, 1}, {15, 1}, {1024, 1}, {1039, 1}, {1040, 2}, {12301, 12}};
+  for (const auto& t : odd)
+    expect(marked_shape(t[0], 100, 1, false).units_per_chunk == t[1], "unaligned units");
   if (failures) {
     std::printf("%d checks failed\n", failures);
     return 1;

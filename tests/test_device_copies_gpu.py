@@ -67,8 +67,10 @@ def bases(layers, base):
 # many units; layers of none, one and several blocks.
 MARKED = [(bpb, 2, (3, 0, 1, 17), 40, cap)
           for bpb in (16, 1008, 1024, 1040, 2032, 2048, 2064, 8208, 36864) for cap in (0, 3)]
-# A launch large enough for the larger share of a workgroup, blocks-first and split.
+# Launches large enough for the larger shares of a workgroup, blocks-first and split.
 MARKED += [(32768, 2, (300, 301), 400, 0), (36864, 1, (511, 1, 512), 600, 0)]
+# A launch with a workgroup's middle share (layers of 2 MiB and more, or 32 MiB in all).
+MARKED += [(4096, 1, (700,), 800, 0), (36864, 1, (100, 99) * 5, 120, 7)]
 # More layers than a workgroup has lanes.
 MARKED += [(1040, 2, (1, 0, 3) * 180, 20, 0), (1040, 2, (1, 0, 3) * 180, 20, 5)]
 
