@@ -512,7 +512,8 @@ int pf_load_layers_noalloc(pf_stream stream, const pf_layer_xfer* layers,
  * the rest is planned) and its last workgroup on layer l writes the marks of
  * layer l.  Layers whose chunks are not all 16-byte aligned share a launch too,
  * marked as they land out of device memory, after the launch out of pinned host
- * memory; DMA copies are marked after each layer's copies.  In PF_MODE_STAGED
+ * memory.  Layers of 96 MiB and more out of device memory have a launch each,
+ * followed by their marks; DMA copies are marked after each layer's copies.  In PF_MODE_STAGED
  * (and AUTO when it stages) each slice's scatter marks the layers it completes, counting a
  * layer's tiles over the slices that hold it, so a layer lands after one
  * kernel; layers in slices that cannot carry them (more than 8 layers,

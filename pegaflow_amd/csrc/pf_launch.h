@@ -34,6 +34,15 @@ inline bool table_in_place(size_t n, uint64_t chunk_bytes, bool is_save) {
 // chunk share its read, so few chunks cost little: 32 of 8 MiB -5.5.
 inline bool waves_in_place(size_t n, uint64_t narrow) { return n <= 64 || narrow <= 64ull << 20; }
 
+// A marked load's layers from device memory share one launch that marks each as it
+// lands, but for layers of this size: those have a fixed-map launch each, and their
+// marks behind it.  The marked kernel falls behind that by a fifth once a call
+// exceeds the memory-side cache (256 MiB), and the launches cost about 8 us a layer.
+// One launch and one a layer, us a call: 8 layers of 32 MiB 105 and 146, of 64 MiB
+// 238 and 228 (by 32 KiB chunks 252 and 256), of 96 MiB 347 and 316 (362 and 351), of
+// 128 MiB 461 and 402 (469 and 453), of 256 MiB 874 and 725.
+constexpr uint64_t kOwnLaunchBytes = 96ull << 20;
+
 // Workgroups of a load of n chunks in place on a route at its default grid.  Each
 // reads the whole table first, and a load of few bytes has no work for many:
 // with 16 and 64 workgroups, 2 MiB (64 chunks of 32 KiB) load in 61.7 and 65.3 us,

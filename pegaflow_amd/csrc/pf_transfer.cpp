@@ -1687,7 +1687,11 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     bytes += plans[li].chunks.size() * plans[li].chunk_bytes;
   }
   // Without per-layer events, consecutive layers with the same chunk size and
-  // alignment share one launch (marks keep per-layer completion inside it).
+  // alignment share one launch (marks keep per-layer completion inside it), but
+  // for large marked ones out of device memory.
+  auto own_launch = [&](const LayerPlan& p) {
+    return sig && p.chunks.size() * p.chunk_bytes >= kOwnLaunchBytes && !host_sourced(p, is_save);
+  };
   std::vector<Step> steps;
   // Marked launches: chunk_start[n+1], then layer[n], then (device copies) wg_start[n+1].
   std::vector<uint32_t> aux;
@@ -1703,17 +1707,18 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     // aligned), and a marked device copy when they are device memory: one
     // launch holds layers of one kind.
     const bool host_src = !p.chunks.empty() && host_sourced(p, is_save);
+    const bool own = layer_events || own_launch(p);
     size_t lj = li + 1;
-    if (!layer_events) {
+    if (!own) {
       while (lj < plans.size() && !plans[lj].ordered &&
              plans[lj].chunk_bytes == p.chunk_bytes &&
              (plans[lj].chunks.empty() ||
-              (chunks_aligned(plans[lj]) == al &&
+              (chunks_aligned(plans[lj]) == al && !own_launch(plans[lj]) &&
                (!sig || host_sourced(plans[lj], is_save) == host_src))))
         ++lj;
     }
     Step st{li, lj, false, al};
-    if (sig && (al || !host_src) && p.chunk_bytes > 0 && !layer_events) {
+    if (sig && (al || !host_src) && p.chunk_bytes > 0 && !own) {
       st.tab = aux.size();
       size_t chunks = 0, groups = 0;
       for (size_t k = li; k < lj; ++k) {
@@ -1841,8 +1846,8 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     if (layer_events && layer_events[st.li])
       PF_HIP(hipEventRecord(static_cast<hipEvent_t>(layer_events[st.li]), x->stream));
     if (sig) {
-      // Layers the launch did not mark: empty ones, and all of an unaligned launch
-      // over the host link or of one with no bytes to copy.
+      // Layers the launch did not mark: empty ones, large ones out of device memory,
+      // and all of an unaligned launch over the host link or of one with no bytes.
       std::vector<uint32_t> rest;
       for (size_t k = st.li; k < st.lj; ++k)
         if (!marked || plans[k].chunks.empty())

@@ -102,6 +102,30 @@ def test_marked_load_from_device_memory(gpu, bpb, segs, counts, nb, cap):
     ctx.close()
 
 
+@pytest.mark.parametrize("bpb", [65536, 65537])
+def test_large_marked_layers_have_a_launch_each(gpu, bpb):
+    """Layers of 96 MiB and more among smaller and empty ones: every byte, every word, and
+    the copies that it took."""
+    counts = (2, 800, 0, 1, 767, 768)  # 96 MiB are 768 blocks of 2 x 64 KiB
+    layers = make_layers(np.random.default_rng(bpb), bpb, 2, counts, 804)
+    pool, words = DeviceBuffer(sum(l.nbytes for l in layers)), PinnedBuffer(8 * len(layers))
+    pool.fill_random(4, nbytes=pool.nbytes // 8 * 8)
+    packed = pool.download()
+    words.array[:] = 0
+    ctx = TransferContext(0)
+    for value in (1, 2):
+        ctx.load_layers_marked([l.transfer(b) for l, b in zip(layers, bases(layers, pool.ptr))],
+                               [(words.ptr, value, True)], _lib.MODE_KERNEL)
+        ctx.synchronize()
+        assert words.array.view(np.uint64).tolist() == [value] * len(layers)
+        # The first layer; the second; the next three; the last.
+        assert ctx.last_stats()[0] == 4
+    for l, at in zip(layers, bases(layers, 0)):
+        l.restore(packed[at:at + l.nbytes])
+        assert np.array_equal(l.dev.download(), l.host)
+    ctx.close()
+
+
 # Chunks around a wave's words and its units at each number of loads per lane,
 # a last unit of one word, and launches of one chunk.
 FIXED = [(bpb, segs, n) for bpb in (16, 1008, 1024, 1040, 4096, 10240, 16400) for segs, n in

@@ -305,13 +305,13 @@ def test_layers_of_zero_byte_blocks_are_marked(gpu, pool):
 
 
 class MarkedCopies:
-    """8 layers of 1,000 blocks each (2 x 64 KiB, or a byte more) out of a pool into
-    tensors of 1,100: in random order, but for the last 16, whose places in the layer's
-    second segment are its end, as they are in the pool."""
+    """8 layers of n blocks each (2 x 64 KiB, or a byte more) out of a pool into tensors
+    of 100 more: in random order, but for the last 16, whose places in the layer's second
+    segment are its end, as they are in the pool."""
 
-    def __init__(self, pool, bpb):
+    def __init__(self, pool, bpb, n):
         rng = np.random.Generator(np.random.PCG64(bpb))
-        nb, n, self.layers, self.tail = 1100, 1000, 8, 16 * bpb
+        nb, self.layers, self.tail = n + 100, 8, 16 * bpb
         self.pool, self.payload = pool(8 * 2 * n * bpb), 2 * n * bpb
         self.bufs = [DeviceBuffer((2 * nb * bpb + 7) // 8 * 8) for _ in range(self.layers)]
         self.end, self.ids = 2 * nb * bpb, []
@@ -346,22 +346,24 @@ class MarkedCopies:
             b.close()
 
 
-MARKED_COPIES = {"device": (DeviceBuffer, 65536, "kernel"),
-                 "device_unaligned": (DeviceBuffer, 65537, "kernel"),
-                 "staged": (PinnedBuffer, 65536, "staged")}
+# The last kind's layers, of 131 MB, have a launch each.
+MARKED_COPIES = {"device": (DeviceBuffer, 65536, 700, "kernel"),
+                 "device_unaligned": (DeviceBuffer, 65537, 700, "kernel"),
+                 "staged": (PinnedBuffer, 65536, 700, "staged"),
+                 "device_large": (DeviceBuffer, 65536, 1000, "kernel")}
 
 
 @pytest.mark.parametrize("kind", list(MARKED_COPIES))
 def test_marked_copies_land_layer_by_layer(gpu, kind):
-    """A load of 1 GB whose copies mark their layers themselves: the host sees the first
-    layer's word while the last one's is not set (0.3 ms later at the least), and a consumer
+    """A load of 0.7 GB whose copies mark their layers themselves: the host sees the first
+    layer's word while the last one's is not set (0.1 ms later at the least), and a consumer
     stream that waits on each layer's device word finds the last bytes that the copy wrote
-    of it (a layer is 131 MB: what the kernel has not yet written, or has left in some L2,
+    of it (a layer is 92 MB: what the kernel has not yet written, or has left in some L2,
     would be missing)."""
     say(f"[gpu] marked copies, layer by layer: {kind}")
-    pool, bpb, mode = MARKED_COPIES[kind]
+    pool, bpb, n, mode = MARKED_COPIES[kind]
     x = TransferContext(0, staging_bytes=512 * MiB if mode == "staged" else 0)
-    c = MarkedCopies(pool, bpb)
+    c = MarkedCopies(pool, bpb, n)
     L = c.layers
     host_words, dev_words, flag = PinnedBuffer(8 * L), DeviceBuffer(8 * L), DeviceBuffer(4 * L)
     snaps = [DeviceBuffer(c.tail) for _ in range(L)]
