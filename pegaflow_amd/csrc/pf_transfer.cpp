@@ -448,9 +448,14 @@ struct pf_xfer {
   // part, i.e. once every earlier launch (a reader of the descriptors) ended.
   hipEvent_t parts_ready = nullptr;
   // Small calls: descriptors the kernels read in place from coherent pinned
-  // memory (kHostDescMax entries), reused only once the stream has drained.
+  // memory (kHostDescMax entries), reused only once the stream has drained:
+  // small_inflight from a call that reads them until the stream was found idle
+  // (calls counts the calls, so that a wait knows of later ones).  busy_until:
+  // when the kernels issued last are expected to have ended.
   ChunkDesc* h_small = nullptr;
   bool small_inflight = false;
+  uint64_t calls = 0;
+  std::chrono::steady_clock::time_point busy_until;
   // The upload kernel's own descriptor, read in place: [0] for a call's
   // first part, [1] for a pipelined call's second part.
   ChunkDesc* h_boot = nullptr;
@@ -598,9 +603,16 @@ constexpr size_t kHostDescMax = 2048;
 
 // The in-place buffer for a call of n descriptors, or null when the call
 // must upload (too many, or the previous in-place call may still be read).
+// Asking a stream that is busy puts a marker on it, in front of this call's
+// kernels, for 15-30 us: it is asked only when its kernels have had their time
+// and nobody has waited for them (pf_xfer_synchronize, a blocking save).  Four
+// loads of 1,024 chunks between device buffers, one after another: 142 us with
+// the question, 111 without; a marked load of 672 chunks out of pinned memory,
+// its words awaited, call after call: 266 and 242.
 ChunkDesc* small_desc(pf_xfer* x, size_t n) {
   if (n > kHostDescMax || !x->h_small) return nullptr;
   if (x->small_inflight) {
+    if (std::chrono::steady_clock::now() < x->busy_until) return nullptr;
     if (hipStreamQuery(x->stream) != hipSuccess) {
       (void)hipGetLastError();  // still running (or an error the sync reports)
       return nullptr;
@@ -608,6 +620,14 @@ ChunkDesc* small_desc(pf_xfer* x, size_t n) {
     x->small_inflight = false;
   }
   return x->h_small;
+}
+
+// Kernels and copies of `bytes` bytes have been issued: 40 GB/s over the host link,
+// 1 TB/s between device buffers, and 100 us.
+void issued(pf_xfer* x, uint64_t bytes, bool host_link) {
+  const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(100) +
+                   std::chrono::nanoseconds(bytes / (host_link ? 40 : 1000));
+  x->busy_until = std::max(x->busy_until, end);
 }
 
 // One gather/scatter launch of the n chunks at descs on `stream`.  With
@@ -964,6 +984,12 @@ void for_each_step_chunk(const std::vector<LayerPlan>& plans, const StagedPlan& 
   }
 }
 
+uint64_t staged_bytes(const StagedPlan& sp) {
+  uint64_t bytes = 0;
+  for (const StagedStep& st : sp.steps) bytes += st.n_chunks * st.chunk_bytes;
+  return bytes;
+}
+
 // Every layer of a staged step has its chunks 16-byte aligned in HBM.
 bool step_aligned(const std::vector<LayerPlan>& plans, const StagedPlan& sp,
                   const StagedStep& st) {
@@ -1125,6 +1151,7 @@ int staged_engine(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers,
     if (hd == x->h_small) {
       x->desc_base = x->h_small;
       x->small_inflight = true;
+      issued(x, staged_bytes(sp), true);
       return PF_OK;
     }
     if (sp.n_desc > uploaded) {
@@ -1530,6 +1557,7 @@ int staged(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers, bool is
   if (hd == x->h_small) {
     x->desc_base = x->h_small;
     x->small_inflight = true;
+    issued(x, staged_bytes(sp), true);
   } else if (int rc = upload_desc(x, sp.n_desc)) {
     return rc;
   }
@@ -1796,6 +1824,7 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
     if (used) *used = total + aux_desc;
   }
   if (sure && !sure()) return kNotSure;
+  bool host_link = false;
   const uint32_t* d_aux = reinterpret_cast<const uint32_t*>(x->desc_base + total);
   for (const Step& st : steps) {
     if (st.dma) {
@@ -1839,6 +1868,7 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
           host_side = host_side_pinned(plans[k]);
           break;
         }
+      host_link |= host_side;
       if (int rc = launch(x, first[st.li], n, plans[st.li].chunk_bytes, st.aligned, is_save,
                           host_side, marked ? &marks : nullptr, nullptr, sure != nullptr))
         return rc;
@@ -1855,7 +1885,12 @@ int kernel_direct(pf_xfer* x, const pf_layer_xfer* layers, const std::vector<Lay
       if (int rc = mark_layers(x, rest, *sig)) return rc;
     }
   }
-  if (is_save && wait_save) PF_HIP(hipStreamSynchronize(x->stream));
+  if (is_save && wait_save) {
+    PF_HIP(hipStreamSynchronize(x->stream));
+    x->small_inflight = false;
+  } else {
+    issued(x, bytes, host_link);
+  }
   return PF_OK;
 }
 
@@ -2001,6 +2036,7 @@ int run(pf_xfer* x, const pf_layer_xfer* layers, uint32_t num_layers, uint32_t m
   std::lock_guard<std::mutex> lk(x->mu);
   x->last_kernels = 0;
   x->last_dma = 0;
+  ++x->calls;
   x->ranges = RangeCache();
   PF_HIP(hipSetDevice(x->device));
   const int rc =
@@ -2533,8 +2569,17 @@ pf_stream pf_xfer_stream(pf_xfer* x) { return x ? x->stream : nullptr; }
 
 int pf_xfer_synchronize(pf_xfer* x) {
   if (!x) return fail(PF_ERR_INVALID_ARGUMENT, "null transfer context");
+  // What this wait says of the in-place descriptors holds for the calls that had
+  // issued all their work before it; with another thread's call under way, nothing.
+  std::unique_lock<std::mutex> lk(x->mu, std::try_to_lock);
+  const uint64_t calls = lk.owns_lock() ? x->calls : 0;
+  if (lk.owns_lock()) lk.unlock();
   PF_HIP(hipStreamSynchronize(x->dma));
   PF_HIP(hipStreamSynchronize(x->stream));
+  if (calls > 0 && lk.try_lock()) {
+    if (x->calls == calls) x->small_inflight = false;
+    lk.unlock();
+  }
   return engine_drain(x);
 }
 

@@ -8,11 +8,13 @@ descriptor table that small calls read in place, and of a launch.  The expected
 bytes are a numpy indexing of the same layout.
 """
 
+import threading
+
 import numpy as np
 import pytest
 
 from pegaflow_amd import _lib
-from pegaflow_amd.runtime import DeviceBuffer, PinnedBuffer
+from pegaflow_amd.runtime import DeviceBuffer, PinnedBuffer, host_wait_word
 from pegaflow_amd.transfer import (KVCacheRegistration, LayerTransfer, TransferContext,
                                    block_array)
 
@@ -289,6 +291,58 @@ def test_scatter_trials_time_no_first_part(gpu, first, rest, timed):
     for l, at in zip(layers, bases(layers, 0)):
         l.restore(packed[at:at + l.nbytes])
         assert np.array_equal(l.dev.download(), l.host)
+    ctx.close()
+
+
+@pytest.mark.parametrize("memory", [PinnedBuffer, DeviceBuffer])
+def test_small_calls_one_after_another(gpu, memory):
+    """Loads whose descriptors may be read in place, each of its own blocks into its own:
+    one behind another with no wait, after a wait, behind marks that were awaited, and
+    from two threads that share the context and wait on their own."""
+    (layer,) = make_layers(np.random.default_rng(1), 4096, 2, (64,), 6000)
+    n, words = 60, PinnedBuffer(8)
+    words.array[:] = 0
+    ids = np.random.default_rng(2).permutation(6000)[:n * 64].reshape(n, 64)
+    pool = memory(n * layer.nbytes)
+    packed = np.random.default_rng(3).integers(0, 256, pool.nbytes, np.uint8)
+    if memory is PinnedBuffer:
+        pool.array[:] = packed
+    else:
+        pool.upload(packed)
+    ctx = TransferContext(0)
+
+    def load(i, marked=False):
+        layer.ids = ids[i]
+        xfer = [layer.transfer(pool.ptr + i * layer.nbytes)]
+        if marked:
+            ctx.load_layers_marked(xfer, [(words.ptr, i + 1, True)], _lib.MODE_KERNEL)
+            assert host_wait_word(words.ptr, i + 1)
+        else:
+            ctx.load_layers(xfer, _lib.MODE_KERNEL)
+
+    for i in range(20):
+        load(i, marked=i % 5 == 4)
+        if i in (3, 9, 10, 16):
+            ctx.synchronize()
+    lock = threading.Lock()
+
+    def worker(first):
+        for i in range(first, n, 2):
+            with lock:  # the layer's ids; the wait is outside
+                load(i)
+            if i % 3 == 0:
+                ctx.synchronize()
+
+    threads = [threading.Thread(target=worker, args=(first,)) for first in (20, 21)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    ctx.synchronize()
+    for i in range(n):
+        layer.ids = ids[i]
+        layer.restore(packed[i * layer.nbytes:(i + 1) * layer.nbytes])
+    assert np.array_equal(layer.dev.download(), layer.host)
     ctx.close()
 
 
