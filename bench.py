@@ -219,7 +219,7 @@ def leg_interference(layers, saved, loads, P, reps=3):
     for _ in range(3):
         victim()
     solo = statistics.median([victim() for _ in range(20)])
-    out = {"victim": "256 MiB device-to-device copy (chunk kernel, 512 threads)",
+    out = {"victim": "256 MiB device-to-device copy (chunk kernel, 256 threads)",
            "victim_solo_ms": round(solo, 4)}
     ops = {
         "kernel_save": lambda: xt.save_layers(saved, _lib.MODE_KERNEL),
@@ -1596,7 +1596,7 @@ def profile_kernels(kind, seed):
                 tensors (2P);
       scatter_sets: two sets of the 32 layer tensors (42 GB each), A and B:
                 gathers from A, A, B, B, then scatters into A, B, A, B in
-                round-robin order (512 threads, 1 load per lane) and
+                round-robin order (1 load per lane) and
                 A, B, A, B in XCD-major order (2 loads per lane), then one
                 more into A, which is checked;
       zerocopy: the prefix saved to pinned host memory, then restored from
@@ -2296,8 +2296,8 @@ def main():
             "frac": round(gather_gbps / HBM_PEAK_GBPS, 4),
             "traffic": gather_traffic,
             "traffic_source": gather_traffic_src,
-            "kernel": "copy_chunks_v16_kernel<1,nt,nt> 512 threads (device gather: 40960 "
-                      "chunks of 32 KiB, 1 launch)",
+            "kernel": "copy_chunks_v16_kernel<1,nt,through> 256 threads (device gather: 40960 "
+                      "chunks of 32 KiB, 2 launches per call)",
             "bytes_per_launch": 2 * P,
             "ms_per_launch": round(gather_ms, 4),
             "plain_copy_gbps": round(plain_gbps, 1),
@@ -2307,12 +2307,12 @@ def main():
                            "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                            "frac": round(scatter_gbps / HBM_PEAK_GBPS, 4),
                            "traffic": scatter_traffic, "traffic_source": scatter_traffic_src,
-                           "kernel": f"copy_chunks_v16_kernel<{s_unroll & 0xff},nt,nt> "
-                                     f"{s_threads} threads, "
+                           "kernel": f"copy_chunks_v16_kernel<{s_unroll & 0xff},nt,through> "
+                                     f"{min(s_threads, 256)} threads, "
                                      f"{'XCD-major' if s_unroll & _lib.KERNEL_XCD_MAJOR else 'round-robin'}"
                                      " tile order, chosen by the context from two timed "
                                      f"candidates (decided: {s_decided}) (device scatter: "
-                                     "packed HBM -> 640 blocks)",
+                                     "packed HBM -> 640 blocks, 2 launches per call)",
                            "bytes_per_launch": 2 * P, "ms_per_launch": round(scatter_ms, 4)},
         "d2d_memcpy_gbps": round(d2d_gbps, 1),
         "interference": interference,

@@ -321,11 +321,12 @@ int pf_xfer_synchronize(pf_xfer* xfer);
  * hardware's round-robin deal (only with an uncapped grid). */
 #define PF_KERNEL_XCD_MAJOR 0x400u
 /* Scatters only (PF_ROUTE_LOAD_DEVICE): choose the shape on evidence.  The
- * context times two candidate shapes, 512 threads with 2 loads per lane in
- * XCD-major order and 512 threads with 1 load per lane in round-robin order
- * (both non-temporal), twice each on its first scatters of at least 64 MiB,
- * and keeps the faster.  Which one wins depends on where the destination
- * tensors lie in HBM.  The other bits of the value are then ignored. */
+ * context times two candidate shapes, 2 loads per lane in XCD-major order and 1
+ * load per lane in round-robin order (both streaming, both set to 512 threads,
+ * of which a fixed-map launch uses 256), twice each on its first scatters of at
+ * least 64 MiB, and keeps the faster; the first part of a call issued in two is
+ * not timed.  Which one wins depends on where the destination tensors lie in
+ * HBM.  The other bits of the value are then ignored. */
 #define PF_KERNEL_AUTO 0x800u
 /* Launch shapes are kept per route: the direction, and whether the far side
  * of the copy is device memory (an HBM-bound gather or scatter) or pinned
@@ -357,13 +358,15 @@ enum {
  * carries PF_KERNEL_AUTO, and ends it otherwise. */
 int pf_xfer_set_kernel_shape_dir(pf_xfer* xfer, uint32_t direction,
                                  uint32_t threads, uint32_t unroll);
-/* The shape a route's next fixed-map launch uses: the route's setting, or for
- * a scatter route on PF_KERNEL_AUTO the chosen candidate once both have been
- * timed (*decided = 1), else the first candidate (*decided = 0). */
+/* The shape a route's next launch is set to (a fixed-map launch runs at most 256
+ * of the threads in a workgroup): the route's setting, or for a scatter route on
+ * PF_KERNEL_AUTO the chosen candidate once both have been timed (*decided = 1),
+ * else the first candidate (*decided = 0). */
 int pf_xfer_route_shape(pf_xfer* xfer, uint32_t route, uint32_t* threads,
                         uint32_t* unroll, int* decided);
-/* Work distribution per route.  0: one workgroup per tile, dealt to the XCDs
- * by the hardware (best for HBM-bound copies).  N > 0: N persistent
+/* Work distribution per route.  0: a fixed map, one unit of 1 KiB times the loads
+ * per lane a wave, dealt to the XCDs by the hardware (best for HBM-bound copies;
+ * unaligned chunks always run so).  N > 0: N persistent
  * workgroups take tiles from a queue in order (best over the host link,
  * whose bandwidth the XCDs do not share fairly: the queue keeps tiles, and
  * a marked load's layers, finishing in order, and few requests in flight
@@ -379,8 +382,8 @@ int pf_xfer_route_shape(pf_xfer* xfer, uint32_t route, uint32_t* threads,
 #define PF_LOAD_HOST_DEFAULT_GRID 64u
 int pf_xfer_set_route_grid(pf_xfer* xfer, uint32_t route, uint32_t workgroups);
 int pf_xfer_set_kernel_shape(pf_xfer* xfer, uint32_t threads, uint32_t unroll);
-/* Upper bound on workgroups per gather/scatter launch (0 = one workgroup per
- * tile, the default); with a bound, each workgroup loops over tiles. */
+/* Upper bound on workgroups per gather/scatter launch (0 = none, the default);
+ * with a bound, each workgroup of a fixed map loops over its units. */
 int pf_xfer_set_max_grid(pf_xfer* xfer, uint32_t max_workgroups);
 /* The copy engines (HSA SDMA engine id bits, from hsa_amd_sdma_engine_id_t)
  * the staged mode's copies run on for `device`: device to host, then host to

@@ -406,12 +406,12 @@ bool aligned16(uint64_t v) { return (v & 15u) == 0; }
 }  // namespace
 
 // Scatter shapes a context chooses between (route PF_ROUTE_LOAD_DEVICE with
-// PF_KERNEL_AUTO).  Which is faster depends on where the destination tensors
-// lie in HBM: measured into two sets of the 32 Llama layer tensors in one
-// process, the first took 0.417 ms into one set and 0.498 ms into the other,
-// the second 0.463 and 0.475 ms; the bytes moved are the same (every write a
-// full 64 B request).  So a context times both on its first large scatters
-// and keeps the faster.
+// PF_KERNEL_AUTO; a fixed-map launch uses 256 of the threads).  Which is faster
+// depends on where the destination tensors lie in HBM: three quarters of the
+// Llama prefix took 367 us with the first and 345 with the second in one process,
+// and in others the first wins; the bytes moved are the same (every write a full
+// 64 B request).  So a context times both on its first large scatters and keeps
+// the faster.
 constexpr uint32_t kScatterShapes[2][2] = {
     {512, 2u | PF_KERNEL_NONTEMPORAL | PF_KERNEL_XCD_MAJOR},
     {512, 1u | PF_KERNEL_NONTEMPORAL}};
